@@ -435,8 +435,7 @@ int horfft_fwd(lsb_ctx* c, const HorPlan& hp, const double* const* phys, double*
     prof_mark_begin(c, PC_FFT, s, &tok, fft_flops(hp, nf, nplanes), fft_bytes(hp, nf, nplanes, 8, 8));
     const int nrows = nplanes * ny;
     if (fast_fft_len(lh)) {
-        LSB_TRY((fast_xfwd<double, double, double>(in, out, nrows, nf, lh, nxpp, nx, (const cpx<double>*)hp.tw_x,
-                                                   (const cpx<double>*)hp.tw_r, s)));
+        LSB_TRY(fast_xfwd(in, out, nrows, nf, lh, nxpp, nx, (const cpx<double>*)hp.tw_x, (const cpx<double>*)hp.tw_r, s));
     } else {
         int lines = lines_for(lh, sizeof(cpx<double>));
         size_t shm = 2 * (size_t)lines * lh * sizeof(cpx<double>);
@@ -447,8 +446,7 @@ int horfft_fwd(lsb_ctx* c, const HorPlan& hp, const double* const* phys, double*
     }
     const double scale = 1.0 / (double)(nx * ny);
     if (fast_fft_len(ny)) {
-        LSB_TRY((fast_yfwd<double, double, double>(out, out, nplanes, nf, lh, ny, (const cpx<double>*)hp.tw_y, scale,
-                                                   s, c->tune[TUNE_YFWD_F64])));
+        LSB_TRY(fast_yfwd(out, out, nplanes, nf, lh, ny, (const cpx<double>*)hp.tw_y, scale, s, c->tune[TUNE_YFWD_F64]));
     } else {
         int cols = lines_for(ny, sizeof(cpx<double>));
         size_t shm = 2 * (size_t)cols * ny * sizeof(cpx<double>);
@@ -463,9 +461,25 @@ int horfft_fwd(lsb_ctx* c, const HorPlan& hp, const double* const* phys, double*
 }
 
 bool horfft_has_ops(const HorPlan& hp) { return fast_fft_len(hp.ny) && fast_fft_len(hp.lh); }
+bool horfft_needs_stage(const HorPlan& hp) { return pow2_fft_len(hp.ny) && pow2_fft_len(hp.lh); }
+
+// Whether the plain inverse stages its y pass in a compact buffer.  Powers of two always
+// have.  The lengths with a factor 3 or 5 transform in place in the padded rows, as the
+// LDS path does, while the fields stay in the 256 MB last-level cache (240 x 114 x 120, 3
+// fields: 59 us against 56 us staged; 480 x 193 x 240, 1 field: 128 against 142), and
+// stage above it (3 fields: 385 us against 550); also in place where the buffer would
+// have to be allocated under a stream capture or while an ensemble's graphs hold it.
+static bool inv_staged(const lsb_ctx* c, const HorPlan& hp, size_t bytes, hipStream_t s) {
+    if (horfft_needs_stage(hp)) return true;
+    if (bytes <= (size_t)256 << 20) return false;
+    if (c->stage_bytes.size() > 8 && c->stage_bytes[8] >= bytes) return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess) return false;
+    return cs == hipStreamCaptureStatusNone && !c->stage_locked;
+}
 
 int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, double* const* phys, int nf,
-                   int nplanes, const int* ops, hipStream_t s, double* scratch) {
+                   int nplanes, const int* ops, hipStream_t s, double* scratch, bool in_place) {
     if (nf < 1 || nf > kMaxFields) {
         set_error("horfft: 1..16 fields per launch");
         return LSB_E_ARG;
@@ -481,30 +495,29 @@ int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, dou
         any_op = any_op || fo.op[f] != FOP_NONE;
     }
     if (any_op && !horfft_has_ops(hp)) {
-        set_error("horfft: derivative-on-load needs power-of-two nx/2 and ny in 16..256");
+        set_error("horfft: derivative-on-load needs register-resident lengths nx/2 and ny");
         return LSB_E_UNSUPPORTED;
     }
     int tok = -1;
     prof_mark_begin(c, PC_FFT, s, &tok, fft_flops(hp, nf, nplanes), fft_bytes(hp, nf, nplanes, 8, 8));
     const int nrows = nplanes * ny;
-    if (horfft_has_ops(hp)) {
+    const size_t per = (size_t)nplanes * ny * nx;
+    if (horfft_has_ops(hp) && !in_place && (scratch || inv_staged(c, hp, per * nf * sizeof(double), s))) {
         // y pass into a compact scratch (rows of lh complex, 128-byte aligned), then the
         // x pass out of place into the padded physical rows
         void* scr = scratch;
-        const size_t per = (size_t)nplanes * ny * nx;
         if (!scr) LSB_TRY(stage_get(c, 8, per * nf * sizeof(double), &scr));
         FieldList<double> mid{};
         for (int f = 0; f < nf; ++f) mid.p[f] = (double*)scr + per * f;
-        LSB_TRY((fast_yinv<double, double, double>(in, mid, nplanes, nf, lh, ny, lh, (const cpx<double>*)hp.tw_y, fo,
-                                                   c->d_wavx, c->d_wavy, s)));
-        LSB_TRY((fast_xinv<double, double, double>(mid, out, nrows, nf, lh, nx, nxpp, (const cpx<double>*)hp.tw_x,
-                                                   (const cpx<double>*)hp.tw_r, s)));
+        LSB_TRY(fast_yinv(in, mid, nplanes, nf, lh, ny, lh, (const cpx<double>*)hp.tw_y, fo, c->d_wavx, c->d_wavy, s));
+        LSB_TRY(fast_xinv(mid, out, nrows, nf, lh, nx, nxpp, (const cpx<double>*)hp.tw_x, (const cpx<double>*)hp.tw_r,
+                          s));
         prof_mark_end(c, tok, s);
         return LSB_OK;
     }
     if (fast_fft_len(ny)) {
-        LSB_TRY((fast_yinv<double, double, double>(in, out, nplanes, nf, lh, ny, nxpp / 2, (const cpx<double>*)hp.tw_y,
-                                                   fo, c->d_wavx, c->d_wavy, s)));
+        LSB_TRY(fast_yinv(in, out, nplanes, nf, lh, ny, nxpp / 2, (const cpx<double>*)hp.tw_y, fo, c->d_wavx,
+                          c->d_wavy, s));
     } else {
         int cols = lines_for(ny, sizeof(cpx<double>));
         size_t shm = 2 * (size_t)cols * ny * sizeof(cpx<double>);
@@ -515,8 +528,8 @@ int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, dou
         LSB_HIP(hipGetLastError());
     }
     if (fast_fft_len(lh)) {
-        LSB_TRY((fast_xinv<double, double, double>(out, out, nrows, nf, lh, nxpp, nxpp, (const cpx<double>*)hp.tw_x,
-                                                   (const cpx<double>*)hp.tw_r, s)));
+        LSB_TRY(fast_xinv(out, out, nrows, nf, lh, nxpp, nxpp, (const cpx<double>*)hp.tw_x,
+                          (const cpx<double>*)hp.tw_r, s));
     } else {
         int lines = lines_for(lh, sizeof(cpx<double>));
         size_t shm = 2 * (size_t)lines * lh * sizeof(cpx<double>);
@@ -535,8 +548,7 @@ int horfft_inv(lsb_ctx* c, const HorPlan& hp, const double* const* spec, double*
 }
 
 // ------------------------------------------- mixed form, generic lengths
-// Lengths that are not register-resident (nx/2 or ny with a factor 3 or 5, or outside
-// 16..256) run the mixed form's transforms on the Stockham kernels in FP32.
+// Lengths that are not register-resident (fast_fft_len) run the mixed form's transforms on the Stockham kernels in FP32.
 
 // u, du/dx, du/dy of 3 FP64 spectra rounded to 9 FP32 spectra; the derivatives are
 // taken in FP64 first (derivatives.f90:261-303: i kx f, i ky f).  One thread per
@@ -554,15 +566,6 @@ __global__ void k_grad_spec32(FieldList<double> in, FieldList<float> out, long n
     reinterpret_cast<float2*>(out.p[3 * l])[pr] = make_float2((float)v.x, (float)v.y);
     reinterpret_cast<float2*>(out.p[3 * l + 1])[pr] = make_float2((float)(-wx * v.y), (float)(wx * v.x));
     reinterpret_cast<float2*>(out.p[3 * l + 2])[pr] = make_float2((float)(-wy * v.y), (float)(wy * v.x));
-}
-
-// FP32 spectra widened to FP64, n values per field
-__global__ void k_widen_f32(FieldList<float> in, FieldList<double> out, long n, int nf) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * nf) return;
-    const int f = (int)(t / n);
-    const long i = t - (long)f * n;
-    out.p[f][i] = (double)in.p[f][i];
 }
 
 // inverse y pass then x pass of nf FP32 spectra into padded FP32 physical rows
@@ -655,8 +658,8 @@ int horfft_inv_grad(lsb_ctx* c, const HorPlan& hp, const double* const* uif, RT*
         if constexpr (sizeof(RT) == 4) {
             if (!ftab) return inv_grad32_generic(c, hp, uif, u, dudx, dudy, nplanes, s);
         }
-        set_error("horfft: the fused FP64 gradient transform and the filter on load need power-of-two nx/2 and ny "
-                  "in 16..256");
+        set_error("horfft: the fused FP64 gradient transform and the filter on load need register-resident lengths "
+                  "nx/2 and ny");
         return LSB_E_UNSUPPORTED;
     }
     const int nx = hp.nx, ny = hp.ny, lh = hp.lh, nxpp = nx + 2;
@@ -681,9 +684,9 @@ int horfft_inv_grad(lsb_ctx* c, const HorPlan& hp, const double* const* uif, RT*
     const cpx<RT>* twy = (const cpx<RT>*)(sizeof(RT) == 8 ? (void*)hp.tw_y : (void*)hp.tw_y32);
     const cpx<RT>* twx = (const cpx<RT>*)(sizeof(RT) == 8 ? (void*)hp.tw_x : (void*)hp.tw_x32);
     const cpx<RT>* twr = (const cpx<RT>*)(sizeof(RT) == 8 ? (void*)hp.tw_r : (void*)hp.tw_r32);
-    LSB_TRY((fast_yinv3<RT, double, RT>(in, mid, nplanes, 3, lh, ny, lh, twy, c->d_wavx, c->d_wavy, ftab, s,
-                                        c->tune[sizeof(RT) == 8 ? TUNE_YINV3_F64 : TUNE_YINV3_F32])));
-    LSB_TRY((fast_xinv<RT, RT, RT>(mid, out, nplanes * ny, 9, lh, nx, nxpp, twx, twr, s)));
+    LSB_TRY(fast_yinv3<RT>(in, mid, nplanes, 3, lh, ny, lh, twy, c->d_wavx, c->d_wavy, ftab, s,
+                           c->tune[sizeof(RT) == 8 ? TUNE_YINV3_F64 : TUNE_YINV3_F32]));
+    LSB_TRY(fast_xinv<RT>(mid, out, nplanes * ny, 9, lh, nx, nxpp, twx, twr, s));
     prof_mark_end(c, tok, s);
     return LSB_OK;
 }
@@ -692,60 +695,39 @@ template int horfft_inv_grad<double>(lsb_ctx*, const HorPlan&, const double* con
 template int horfft_inv_grad<float>(lsb_ctx*, const HorPlan&, const double* const*, float* const*, float* const*,
                                     float* const*, int, const double*, hipStream_t);
 
-// Mixed form: FP32 physical fields, FP64 spectra, FP32 arithmetic.
-template <class TO>
-int horfft_fwd_mixed(lsb_ctx* c, const HorPlan& hp, const float* const* phys, TO* const* spec, int nf, int nplanes,
+// Mixed form: FP32 physical fields, FP32 spectra and arithmetic.
+int horfft_fwd_mixed(lsb_ctx* c, const HorPlan& hp, const float* const* phys, float* const* spec, int nf, int nplanes,
                      hipStream_t s) {
     if (nf < 1 || nf > kMaxFields) {
         set_error("horfft (mixed): 1..16 fields per launch");
         return LSB_E_ARG;
     }
     const int nx = hp.nx, ny = hp.ny, lh = hp.lh, nxpp = nx + 2;
-    void* scr = nullptr;
-    const size_t per = (size_t)nplanes * ny * nx;
-    if (!horfft_has_ops(hp)) {
-        // generic lengths: Stockham passes in FP32 (into staging first when the spectra are FP64)
-        FieldList<float> in{}, mid{};
-        FieldList<double> wide{};
-        if (sizeof(TO) == 8) LSB_TRY(stage_get(c, 8, per * nf * sizeof(float), &scr));
-        for (int f = 0; f < nf; ++f) {
-            in.p[f] = const_cast<float*>(phys[f]);
-            mid.p[f] = sizeof(TO) == 8 ? (float*)scr + per * f : reinterpret_cast<float*>(spec[f]);
-            wide.p[f] = reinterpret_cast<double*>(spec[f]);
-        }
-        int tok = -1;
-        prof_mark_begin(c, PC_FFT, s, &tok, fft_flops(hp, nf, nplanes), fft_bytes(hp, nf, nplanes, 4, sizeof(TO)));
-        LSB_TRY(generic_fwd32(hp, in, mid, nf, nplanes, s));
-        if (sizeof(TO) == 8) {
-            hipLaunchKernelGGL(k_widen_f32, dim3((unsigned)(((long)per * nf + 255) / 256)), dim3(256), 0, s, mid, wide,
-                               (long)per, nf);
-            LSB_HIP(hipGetLastError());
-        }
-        prof_mark_end(c, tok, s);
-        return LSB_OK;
-    }
-    LSB_TRY(stage_get(c, 8, per * nf * sizeof(float), &scr));
-    FieldList<float> in{}, mid{};
-    FieldList<TO> out{};
+    FieldList<float> in{}, out{};
     for (int f = 0; f < nf; ++f) {
         in.p[f] = const_cast<float*>(phys[f]);
-        mid.p[f] = (float*)scr + per * f;
         out.p[f] = spec[f];
     }
     int tok = -1;
-    prof_mark_begin(c, PC_FFT, s, &tok, fft_flops(hp, nf, nplanes), fft_bytes(hp, nf, nplanes, 4, sizeof(TO)));
-    const int nrows = nplanes * ny;
-    LSB_TRY((fast_xfwd<float, float, float>(in, mid, nrows, nf, lh, nxpp, nx, (const cpx<float>*)hp.tw_x32,
-                                            (const cpx<float>*)hp.tw_r32, s)));
-    LSB_TRY((fast_yfwd<float, float, TO>(mid, out, nplanes, nf, lh, ny, (const cpx<float>*)hp.tw_y32,
-                                             1.0f / (float)(nx * ny), s, c->tune[TUNE_YFWD_F32])));
+    prof_mark_begin(c, PC_FFT, s, &tok, fft_flops(hp, nf, nplanes), fft_bytes(hp, nf, nplanes, 4, 4));
+    if (!horfft_has_ops(hp)) {
+        // generic lengths: Stockham passes in FP32
+        LSB_TRY(generic_fwd32(hp, in, out, nf, nplanes, s));
+        prof_mark_end(c, tok, s);
+        return LSB_OK;
+    }
+    void* scr = nullptr;
+    const size_t per = (size_t)nplanes * ny * nx;
+    LSB_TRY(stage_get(c, 8, per * nf * sizeof(float), &scr));
+    FieldList<float> mid{};
+    for (int f = 0; f < nf; ++f) mid.p[f] = (float*)scr + per * f;
+    LSB_TRY(fast_xfwd(in, mid, nplanes * ny, nf, lh, nxpp, nx, (const cpx<float>*)hp.tw_x32,
+                      (const cpx<float>*)hp.tw_r32, s));
+    LSB_TRY(fast_yfwd(mid, out, nplanes, nf, lh, ny, (const cpx<float>*)hp.tw_y32, 1.0f / (float)(nx * ny), s,
+                      c->tune[TUNE_YFWD_F32]));
     prof_mark_end(c, tok, s);
     return LSB_OK;
 }
-template int horfft_fwd_mixed<double>(lsb_ctx*, const HorPlan&, const float* const*, double* const*, int, int,
-                                      hipStream_t);
-template int horfft_fwd_mixed<float>(lsb_ctx*, const HorPlan&, const float* const*, float* const*, int, int,
-                                     hipStream_t);
 
 // ------------------------------------------------ y-pass tile autotuning
 // Times the kx-column tiles of the y passes the step uses (forward y pass, the gradient
@@ -754,7 +736,7 @@ template int horfft_fwd_mixed<float>(lsb_ctx*, const HorPlan&, const float* cons
 // zeroed scratch of at least 24 physical fields of doubles.
 int fft_tune_y(lsb_ctx* c, void* work, hipStream_t s) {
     const HorPlan& hp = c->hp;
-    if (!horfft_has_ops(hp)) return LSB_OK;
+    if (!horfft_has_ops(hp) || !pow2_fft_len(hp.ny)) return LSB_OK;  // the other lengths have one tile width
     const int np = c->nzp, lh = hp.lh, ny = hp.ny;
     const size_t nsp = (size_t)np * ny * hp.nx;  // reals of one spectral field
     char* w = static_cast<char*>(work);
@@ -802,12 +784,10 @@ int fft_tune_y(lsb_ctx* c, void* work, hipStream_t s) {
             out32.p[f] = f32(3 + f);
         }
         pick(TUNE_YFWD_F64, "yfwd f64", c64, 2, [&](int cc) {
-            return fast_yfwd<double, double, double>(in, out, np, 3, lh, ny, (const cpx<double>*)hp.tw_y, scale, s,
-                                                     cc);
+            return fast_yfwd<double>(in, out, np, 3, lh, ny, (const cpx<double>*)hp.tw_y, scale, s, cc);
         });
         pick(TUNE_YFWD_F32, "yfwd f32", c32, 3, [&](int cc) {
-            return fast_yfwd<float, float, float>(in32, out32, np, 3, lh, ny, (const cpx<float>*)hp.tw_y32,
-                                                  (float)scale, s, cc);
+            return fast_yfwd<float>(in32, out32, np, 3, lh, ny, (const cpx<float>*)hp.tw_y32, (float)scale, s, cc);
         });
     }
     {   // gradient transform's inverse y pass: 3 FP64 spectra -> 9 fields
@@ -819,11 +799,11 @@ int fft_tune_y(lsb_ctx* c, void* work, hipStream_t s) {
             out32.p[f] = f32(6 + f);  // after the 3 FP64 inputs (6 FP32 fields of room)
         }
         pick(TUNE_YINV3_F64, "yinv3 f64", c64, 2, [&](int cc) {
-            return fast_yinv3<double, double, double>(in, out, np, 3, lh, ny, lh, (const cpx<double>*)hp.tw_y,
+            return fast_yinv3<double>(in, out, np, 3, lh, ny, lh, (const cpx<double>*)hp.tw_y,
                                                       c->d_wavx, c->d_wavy, nullptr, s, cc);
         });
         pick(TUNE_YINV3_F32, "yinv3 f32", c32, 3, [&](int cc) {
-            return fast_yinv3<float, double, float>(in, out32, np, 3, lh, ny, lh, (const cpx<float>*)hp.tw_y32,
+            return fast_yinv3<float>(in, out32, np, 3, lh, ny, lh, (const cpx<float>*)hp.tw_y32,
                                                     c->d_wavx, c->d_wavy, nullptr, s, cc);
         });
     }
@@ -853,7 +833,7 @@ int fft_tune_y(lsb_ctx* c, void* work, hipStream_t s) {
         a.dt = c->dt;
         a.dtnui = 1.0;
         pick(TUNE_YRHS_F32, "yfwd+rhs f32", c32, 3, [&](int cc) {
-            return fast_yfwd_rhs<float, float>(pc, np, lh, ny, (const cpx<float>*)hp.tw_y32, (float)scale, a, s, cc);
+            return fast_yfwd_rhs(pc, np, lh, ny, (const cpx<float>*)hp.tw_y32, (float)scale, a, s, cc);
         });
     }
     (void)hipEventDestroy(e0);
@@ -867,7 +847,7 @@ template <class T>
 int horfft_xfwd(lsb_ctx* c, const HorPlan& hp, const T* const* phys, T* const* rows, int nf, int nplanes,
                 hipStream_t s) {
     if (nf < 1 || nf > kMaxFields || !horfft_has_ops(hp)) {
-        set_error("horfft (x pass): 1..16 fields, power-of-two nx/2 and ny in 16..256");
+        set_error("horfft (x pass): 1..16 fields, register-resident lengths nx/2 and ny");
         return LSB_E_UNSUPPORTED;
     }
     FieldList<T> in{}, out{};
@@ -881,7 +861,7 @@ int horfft_xfwd(lsb_ctx* c, const HorPlan& hp, const T* const* phys, T* const* r
                     planes * ((double)(hp.nx + 2) * hp.ny + (double)hp.nx * hp.ny) * sizeof(T));
     const cpx<T>* twx = (const cpx<T>*)(sizeof(T) == 8 ? (void*)hp.tw_x : (void*)hp.tw_x32);
     const cpx<T>* twr = (const cpx<T>*)(sizeof(T) == 8 ? (void*)hp.tw_r : (void*)hp.tw_r32);
-    LSB_TRY((fast_xfwd<T, T, T>(in, out, nplanes * hp.ny, nf, hp.lh, hp.nx + 2, hp.nx, twx, twr, s)));
+    LSB_TRY(fast_xfwd<T>(in, out, nplanes * hp.ny, nf, hp.lh, hp.nx + 2, hp.nx, twx, twr, s));
     prof_mark_end(c, tok, s);
     return LSB_OK;
 }
@@ -891,65 +871,25 @@ template int horfft_xfwd<float>(lsb_ctx*, const HorPlan&, const float* const*, f
 
 // y pass of the three pieces of each N_l fused with the velocity right-hand side
 // (fast_yfwd_rhs); pieces[3 l + q] hold x-transformed rows.
-template <class R, class TH>
-int horfft_yfwd_rhs(lsb_ctx* c, const HorPlan& hp, R* const* pieces, int nplanes, const YRhsArgs& a, hipStream_t s) {
+int horfft_yfwd_rhs(lsb_ctx* c, const HorPlan& hp, float* const* pieces, int nplanes, const YRhsArgs& a,
+                    hipStream_t s) {
     if (!horfft_has_ops(hp)) {
-        set_error("horfft (fused y pass): power-of-two nx/2 and ny in 16..256");
+        set_error("horfft (fused y pass): register-resident lengths nx/2 and ny");
         return LSB_E_UNSUPPORTED;
     }
-    FieldList<R> pc{};
+    FieldList<float> pc{};
     for (int q = 0; q < 9; ++q) pc.p[q] = pieces[q];
     int tok = -1;
     {
         const double pairs = (double)nplanes * hp.ny * hp.lh * 3.0;
-        const double per = 3.0 * 2 * sizeof(R) + 3.0 * 2 * sizeof(TH) + 4.0 * 16.0;
+        const double per = 3.0 * 2 * sizeof(float) + 3.0 * 2 * sizeof(float) + 4.0 * 16.0;
         prof_mark_begin(c, PC_RHS, s, &tok, 9.0 * nplanes * 2.5 * hp.lh * hp.ny * std::log2((double)hp.ny),
                         pairs * per);
     }
-    const cpx<R>* twy = (const cpx<R>*)(sizeof(R) == 8 ? (void*)hp.tw_y : (void*)hp.tw_y32);
-    LSB_TRY((fast_yfwd_rhs<R, TH>(pc, nplanes, hp.lh, hp.ny, twy, (R)(1.0 / ((double)hp.nx * hp.ny)), a, s,
-                                  sizeof(R) == 4 ? c->tune[TUNE_YRHS_F32] : 0)));
+    LSB_TRY(fast_yfwd_rhs(pc, nplanes, hp.lh, hp.ny, (const cpx<float>*)hp.tw_y32,
+                          (float)(1.0 / ((double)hp.nx * hp.ny)), a, s, c->tune[TUNE_YRHS_F32]));
     prof_mark_end(c, tok, s);
     return LSB_OK;
 }
-template int horfft_yfwd_rhs<double, double>(lsb_ctx*, const HorPlan&, double* const*, int, const YRhsArgs&,
-                                             hipStream_t);
-template int horfft_yfwd_rhs<float, float>(lsb_ctx*, const HorPlan&, float* const*, int, const YRhsArgs&,
-                                           hipStream_t);
-
-template <class TI>
-int horfft_inv_mixed(lsb_ctx* c, const HorPlan& hp, const TI* const* spec, float* const* phys, int nf, int nplanes,
-                     const int* ops, hipStream_t s) {
-    if (nf < 1 || nf > kMaxFields || !horfft_has_ops(hp)) {
-        set_error("horfft (mixed): 1..16 fields, power-of-two nx/2 and ny in 16..256");
-        return LSB_E_UNSUPPORTED;
-    }
-    const int nx = hp.nx, ny = hp.ny, lh = hp.lh, nxpp = nx + 2;
-    void* scr = nullptr;
-    const size_t per = (size_t)nplanes * ny * nx;
-    LSB_TRY(stage_get(c, 8, per * nf * sizeof(float), &scr));
-    FieldList<TI> in{};
-    FieldList<float> mid{}, out{};
-    FftOps fo{};
-    for (int f = 0; f < nf; ++f) {
-        in.p[f] = const_cast<TI*>(spec[f]);
-        mid.p[f] = (float*)scr + per * f;
-        out.p[f] = phys[f];
-        fo.op[f] = ops ? ops[f] : FOP_NONE;
-    }
-    int tok = -1;
-    prof_mark_begin(c, PC_FFT, s, &tok, fft_flops(hp, nf, nplanes), fft_bytes(hp, nf, nplanes, 4, sizeof(TI)));
-    const int nrows = nplanes * ny;
-    LSB_TRY((fast_yinv<float, TI, float>(in, mid, nplanes, nf, lh, ny, lh, (const cpx<float>*)hp.tw_y32, fo,
-                                         c->d_wavx, c->d_wavy, s)));
-    LSB_TRY((fast_xinv<float, float, float>(mid, out, nrows, nf, lh, nx, nxpp, (const cpx<float>*)hp.tw_x32,
-                                            (const cpx<float>*)hp.tw_r32, s)));
-    prof_mark_end(c, tok, s);
-    return LSB_OK;
-}
-template int horfft_inv_mixed<double>(lsb_ctx*, const HorPlan&, const double* const*, float* const*, int, int,
-                                      const int*, hipStream_t);
-template int horfft_inv_mixed<float>(lsb_ctx*, const HorPlan&, const float* const*, float* const*, int, int,
-                                     const int*, hipStream_t);
 
 }  // namespace lsb

@@ -1,0 +1,9 @@
+// The register-resident FFT passes of the lengths with a factor 3 or 5: FP64, x passes.
+#include "fft_fast_kernels.h"
+
+namespace lsb {
+#define X(LL, A, B) LSB_MIXED_X(, double, A, B)
+LSB_MIXED_CASES(X)
+LSB_MIXED_ODD_CASES(X)
+#undef X
+}  // namespace lsb

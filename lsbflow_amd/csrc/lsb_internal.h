@@ -316,16 +316,19 @@ int horfft_inv(lsb_ctx* c, const HorPlan& hp, const double* const* spec, double*
                int nplanes, hipStream_t s);
 // inverse with per-field d/dx, d/dy applied on load (FOP_*); fast lengths only
 bool horfft_has_ops(const HorPlan& hp);
+// whether the inverse has always staged its y pass (powers of two)
+bool horfft_needs_stage(const HorPlan& hp);
 template <class T>
 int horfft_xfwd(lsb_ctx* c, const HorPlan& hp, const T* const* phys, T* const* rows, int nf, int nplanes,
                 hipStream_t s);
 struct YRhsArgs;
-template <class R, class TH>
-int horfft_yfwd_rhs(lsb_ctx* c, const HorPlan& hp, R* const* pieces, int nplanes, const YRhsArgs& a, hipStream_t s);
+int horfft_yfwd_rhs(lsb_ctx* c, const HorPlan& hp, float* const* pieces, int nplanes, const YRhsArgs& a,
+                    hipStream_t s);
 // scratch: the y pass's staging buffer (nf * nplanes * ny * nx doubles) supplied by the
-// caller; null takes the context's staging slot 8 (allocated on first use)
+// caller; null takes the context's staging slot 8 (allocated on first use); in_place: no
+// staging, the y pass writes the padded rows
 int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, double* const* phys, int nf,
-                   int nplanes, const int* ops, hipStream_t s, double* scratch = nullptr);
+                   int nplanes, const int* ops, hipStream_t s, double* scratch = nullptr, bool in_place = false);
 // allocation-free entry points (noalloc.hip): resolve the device address of the
 // file-scope scratch array on `device` (the current device); called by lsb_create
 int noalloc_resolve(int device);
@@ -333,13 +336,9 @@ int noalloc_resolve(int device);
 template <class RT>
 int horfft_inv_grad(lsb_ctx* c, const HorPlan& hp, const double* const* uif, RT* const* u, RT* const* dudx,
                     RT* const* dudy, int nplanes, const double* ftab, hipStream_t s);
-// mixed form: FP32 physical fields, FP64 spectra
-template <class TO>
-int horfft_fwd_mixed(lsb_ctx* c, const HorPlan& hp, const float* const* phys, TO* const* spec, int nf, int nplanes,
+// mixed form: nf FP32 physical fields -> FP32 spectra
+int horfft_fwd_mixed(lsb_ctx* c, const HorPlan& hp, const float* const* phys, float* const* spec, int nf, int nplanes,
                      hipStream_t s);
-template <class TI>
-int horfft_inv_mixed(lsb_ctx* c, const HorPlan& hp, const TI* const* spec, float* const* phys, int nf, int nplanes,
-                     const int* ops, hipStream_t s);
 
 // filters.f90:281-335 specfilter_exp_xy on one mode: rebuilt from its magnitude and
 // phase, fmag*filt*(cos(phase), sin(phase)) with cos(phase) = re/fmag and the phase
@@ -367,24 +366,23 @@ enum { FOP_NONE = 0, FOP_DX = 1, FOP_DY = 2 };
 struct FftOps {
     int op[kMaxFields];
 };
-bool fast_fft_len(int L);
-template <class R, class TI, class TO>
-int fast_xfwd(const FieldList<TI>& in, const FieldList<TO>& out, int nrows, int nf, int lh, int istride,
-              int ostride, const cpx<R>* tw, const cpx<R>* twr, hipStream_t s);
-template <class R, class TI, class TO>
-int fast_xinv(const FieldList<TI>& in, const FieldList<TO>& out, int nrows, int nf, int lh, int istride, int nxpp,
+bool fast_fft_len(int L);  // powers of two 16..256 and most lengths 24..240 with a factor 3 or 5
+bool pow2_fft_len(int L);
+template <class R>
+int fast_xfwd(const FieldList<R>& in, const FieldList<R>& out, int nrows, int nf, int lh, int istride, int ostride,
               const cpx<R>* tw, const cpx<R>* twr, hipStream_t s);
-template <class R, class TI, class TO>
-int fast_yfwd(const FieldList<TI>& in, const FieldList<TO>& out, int nplanes, int nf, int lh, int ny,
-              const cpx<R>* tw, R scale, hipStream_t s, int cols = 0);
-template <class R, class TI, class TO>
-int fast_yinv(const FieldList<TI>& in, const FieldList<TO>& out, int nplanes, int nf, int lh, int ny, int ph,
-              const cpx<R>* tw, const FftOps& ops, const double* wavx, const double* wavy, hipStream_t s,
-              int cols = 0);
+template <class R>
+int fast_xinv(const FieldList<R>& in, const FieldList<R>& out, int nrows, int nf, int lh, int istride, int nxpp,
+              const cpx<R>* tw, const cpx<R>* twr, hipStream_t s);
+template <class R>
+int fast_yfwd(const FieldList<R>& in, const FieldList<R>& out, int nplanes, int nf, int lh, int ny, const cpx<R>* tw,
+              R scale, hipStream_t s, int cols = 0);
+int fast_yinv(const FieldList<double>& in, const FieldList<double>& out, int nplanes, int nf, int lh, int ny, int ph,
+              const cpx<double>* tw, const FftOps& ops, const double* wavx, const double* wavy, hipStream_t s);
 // nsrc spectra -> 3 nsrc outputs (u, du/dx, du/dy per source), one load per source
 // ftab (lh*ny factors, index m + lh*ky) applies the spectral filter on load; null: none
-template <class R, class TI, class TO>
-int fast_yinv3(const FieldList<TI>& in, const FieldList<TO>& out, int nplanes, int nsrc, int lh, int ny, int ph,
+template <class R>
+int fast_yinv3(const FieldList<double>& in, const FieldList<R>& out, int nplanes, int nsrc, int lh, int ny, int ph,
                const cpx<R>* tw, const double* wavx, const double* wavy, const double* ftab, hipStream_t s,
                int cols = 0);
 
@@ -404,8 +402,7 @@ struct YRhsArgs {
     double* rhs[3];
     double ab0, ab1, ab2, bdf0, bdf1, bdf2, dt, dtnui;
 };
-template <class R, class TH>
-int fast_yfwd_rhs(const FieldList<R>& pieces, int nplanes, int lh, int ny, const cpx<R>* tw, R scale,
+int fast_yfwd_rhs(const FieldList<float>& pieces, int nplanes, int lh, int ny, const cpx<float>* tw, float scale,
                   const YRhsArgs& a, hipStream_t s, int cols = 0);
 // times the kx-column tiles of the y passes on this context's grid (scratch `work` of
 // at least 24 physical fields of doubles) and records the fastest in the tuning table

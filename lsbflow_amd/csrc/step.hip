@@ -782,7 +782,7 @@ static int nlterm_phys_mixed(lsb_ctx* c, StepState* S, const double* const* uif,
         if (xonly)
             LSB_TRY(horfft_xfwd<float>(c, c->hp, in, out, n, c->nzp, s));
         else
-            LSB_TRY(horfft_fwd_mixed<float>(c, c->hp, in, out, n, c->nzp, s));
+            LSB_TRY(horfft_fwd_mixed(c, c->hp, in, out, n, c->nzp, s));
     }
     return LSB_OK;
 }
@@ -1014,7 +1014,7 @@ static int update_once(lsb_ctx* c) {
         y.bdf2 = r.bdf2;
         y.dt = r.dt;
         y.dtnui = r.dtnui;
-        LSB_TRY((horfft_yfwd_rhs<float, float>(c, c->hp, pieces, c->nzp, y, s)));
+        LSB_TRY(horfft_yfwd_rhs(c, c->hp, pieces, c->nzp, y, s));
     } else {
         LSB_TRY(sp_rhs_vel(c, r, s));
     }

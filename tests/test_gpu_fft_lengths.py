@@ -1,0 +1,135 @@
+"""The horizontal transforms at the lengths with a factor 3 or 5.
+
+Every x length (nx/2) and y length (ny) of the register-resident passes that is not a
+power of two, one plane count that leaves a partial last block of rows, kx columns that
+leave a partial last tile.  FP64 transforms against numpy's (pocketfft): both round each
+of the log2(N) butterfly levels, relative L2 a few eps, bar 4e-15; the fused gradient
+transform and the products against the oracle's nonlinear term (bar 1e-10, the operator
+bar); the mixed form's fused forward pass and right-hand side against the FP64 step, which
+FP32 rounding of the nonlinear chain leaves within 1e-5.
+"""
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import lsbflow_amd as L
+from lsbflow_amd import _lib
+from lsbflow_amd.core import Config, Context, setup_case
+from oracle import Oracle, OracleConfig
+from tests.conftest import rel_l2
+from tests.test_zz_no_alloc import Hip
+
+pytestmark = pytest.mark.gpu
+
+XLEN = [24, 25, 27, 30, 36, 40, 45, 48, 50, 54, 60, 72, 75, 80, 81, 90, 96, 100, 108, 120, 135, 144, 150, 160, 162, 180,
+        192, 200, 216, 225, 240]
+YLEN = [n for n in XLEN if n % 2 == 0]
+PAIRS = [(2 * m, YLEN[(5 * i) % len(YLEN)]) for i, m in enumerate(XLEN)]
+NZP = 5
+
+
+def test_pairs_cover_every_length():
+    assert {ny for _, ny in PAIRS} == set(YLEN)
+
+
+@pytest.mark.parametrize("nx,ny", PAIRS + [(128, 60), (120, 64), (250, 60), (60, 24)])
+def test_transform_pair(nx, ny):
+    rng = np.random.default_rng(nx * 1000 + ny)
+    with Context(Config(nx=nx, ny=ny, nz=NZP - 1)) as ctx:
+        x = np.zeros((2, NZP, ny, nx + 2))
+        x[..., :nx] = rng.standard_normal((2, NZP, ny, nx))
+        ref = np.fft.fft(np.fft.rfft(x[..., :nx])[..., : nx // 2], axis=-2) / (nx * ny)
+        spec = ctx.fwd(x)
+        ef = rel_l2(spec.reshape(ref.shape + (2,)), np.stack([ref.real, ref.imag], axis=-1))
+        s = rng.standard_normal((2, NZP, ny, nx))
+        full = np.zeros((2, NZP, ny, nx // 2 + 1), dtype=complex)
+        full[..., : nx // 2] = np.fft.ifft(np.ascontiguousarray(s).view(complex), axis=-2, norm="forward")
+        back = ctx.inv(s)
+        ei = rel_l2(back[..., :nx], np.fft.irfft(full, n=nx, norm="forward"))
+        assert np.all(back[..., nx:] == 0.0)
+    print(f"{nx}x{ny}: forward {ef:.1e} inverse {ei:.1e}", flush=True)
+    assert ef < 4e-15 and ei < 4e-15
+
+
+def case_of(nx, ny):
+    return L.cases.CASES["c2_dyn_les"].with_(nx=nx, ny=ny, nz=12, sgsmodel=2, xnu=2e-5, dt=2.5e-4, samp=0.1)
+
+
+@pytest.mark.parametrize("nx,ny", PAIRS[::2] + [(50, 60)])
+def test_nonlinear_term(nx, ny):
+    case = case_of(nx, ny).with_(sgsflag=0)
+    keys = OracleConfig.__dataclass_fields__
+    o = Oracle(OracleConfig(**{k: v for k, v in case.as_dict().items() if k in keys}))
+    o.ubar, o.ubarp, o.ubarpp = L.cases.base_flow(case)
+    uif = np.stack(L.cases.initial_condition(case.with_(pert_rms=0.05)))
+    ref, _ = o.nlterm_skewsym(uif, np.zeros_like(uif[0]), 0)
+    with setup_case(case) as ctx:
+        got = ctx.nlterm_skewsym(uif)
+    e = rel_l2(got, ref)
+    print(f"{nx}x{ny}: nonlinear term {e:.1e}", flush=True)
+    assert e < 1e-10
+
+
+@pytest.mark.parametrize("nx,ny", PAIRS)
+def test_mixed_step_against_fp64(nx, ny):
+    case = case_of(nx, ny)
+    out = []
+    for precision in (0, 1):
+        with setup_case(case, precision=precision) as ctx:
+            ctx.state_set(*L.cases.initial_condition(case))
+            ctx.timestep(4)
+            out.append(ctx.state_get())
+    errs = {k: rel_l2(out[1][k], out[0][k]) for k in ("uf", "vf", "wf", "nlnif")}
+    print(f"{nx}x{ny}: mixed vs FP64 {errs}", flush=True)
+    assert max(errs.values()) < 1e-5
+
+
+def test_noalloc_beyond_its_scratch_stays_accepted():
+    """One field of 480 x 240 x 301 exceeds the 2^25-double scratch: the lengths with a
+    factor 3 or 5 transform in place there, to the staged route's bits."""
+    nx, ny, nz = 480, 240, 300
+    hip, lib = Hip(), _lib.lib()
+    with Context(Config(nx=nx, ny=ny, nz=nz)) as ctx:
+        s = np.random.default_rng(3).standard_normal((nz + 1, ny, nx))
+        spec = hip.alloc(s.nbytes)
+        hip.put(spec, s)
+        got = []
+        for fn in (lib.lsb_horfft_dev, lib.lsb_horfft_dev_noalloc):
+            out = hip.alloc((nz + 1) * ny * (nx + 2) * 8)
+            _lib.check(fn(ctx.h, out, spec, 1, 1, None), "horfft")
+            ctx.synchronize()
+            got.append(hip.get(out, (nz + 1, ny, nx + 2)))
+            assert hip.lib.hipFree(out) == 0
+        assert hip.lib.hipFree(spec) == 0
+    assert np.array_equal(*got)
+
+
+def test_inverse_under_capture_without_staging():
+    """A first inverse transform inside a stream capture allocates nothing at these lengths,
+    also beyond the size from which it stages its y pass (one field of 337 MB): it runs in
+    place in the output rows, and the graph replays to the eager, staged bits."""
+    nx, ny, nz = 480, 240, 365
+    hip, lib = Hip(), _lib.lib()
+    shape = (nz + 1, ny, nx + 2)
+    with Context(Config(nx=nx, ny=ny, nz=nz)) as ctx, Context(Config(nx=nx, ny=ny, nz=nz)) as ref:
+        s = np.random.default_rng(5).standard_normal((nz + 1, ny, nx))
+        spec, out, want = hip.alloc(s.nbytes), hip.alloc(8 * np.prod(shape)), hip.alloc(8 * np.prod(shape))
+        hip.put(spec, s)
+        _lib.check(lib.lsb_horfft_dev(ref.h, want, spec, 1, 1, None), "horfft")
+        ref.synchronize()
+        stream, graph, ex = C.c_void_p(ctx.stream()), C.c_void_p(), C.c_void_p()
+        assert hip.lib.hipStreamBeginCapture(stream, 1) == 0
+        _lib.check(lib.lsb_horfft_dev(ctx.h, out, spec, 1, 1, stream), "horfft")
+        assert hip.lib.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert hip.lib.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+        for _ in range(3):
+            hip.put(out, np.zeros(shape))
+            assert hip.lib.hipGraphLaunch(ex, stream) == 0
+            ctx.synchronize()
+            assert np.array_equal(hip.get(out, shape), hip.get(want, shape))
+        hip.lib.hipGraphExecDestroy(ex)
+        hip.lib.hipGraphDestroy(graph)
+        for p in (spec, out, want):
+            assert hip.lib.hipFree(p) == 0
