@@ -901,21 +901,46 @@ static void zsplit_shape(ZArgs& a, const ZSplitOp& op, bool allow_xrow, int rb, 
     *nw = (a.gblocks + rb - 1) / rb;
 }
 
-template <int MODE>
-static int launch_zs(const ZArgs& a0, const ZSplitOp& op, const FieldList<double>& in, const FieldList<double>& out,
-                     const FieldList<double>& bt, const FieldList<double>& bb, int nf, hipStream_t s) {
+template <int MODE, int RB, int CB, int WPE>
+static int launch_zs_shape(const ZArgs& a0, const ZSplitOp& op, const FieldList<double>& in,
+                           const FieldList<double>& out, const FieldList<double>& bt, const FieldList<double>& bb,
+                           int nf, hipStream_t s) {
     ZArgs a = a0;
     int gy = 1, nw = 1;
-    // two input fields or a wider epilogue: two row blocks per wave keep three waves per SIMD
-    constexpr int RB = (MODE == ZM_PRESSDIV || MODE == ZM_PROJ) ? 2 : kZSRB;
     zsplit_shape(a, op, MODE != ZM_HELM1 && MODE != ZM_HELM2, RB, &gy, &nw);
-    dim3 grid((unsigned)((a.P + 16 * kZSCB - 1) / (16 * kZSCB)), (unsigned)gy, (unsigned)nf);
+    dim3 grid((unsigned)((a.P + 16 * CB - 1) / (16 * CB)), (unsigned)gy, (unsigned)nf);
     if (a.xrow >= 0)
-        hipLaunchKernelGGL((k_zsplit<MODE, true, RB>), grid, dim3(64 * nw), 0, s, a, in, out, bt, bb);
+        hipLaunchKernelGGL((k_zsplit<MODE, true, RB, CB, kZPD, WPE>), grid, dim3(64 * nw), 0, s, a, in, out, bt, bb);
     else
-        hipLaunchKernelGGL((k_zsplit<MODE, false, RB>), grid, dim3(64 * nw), 0, s, a, in, out, bt, bb);
+        hipLaunchKernelGGL((k_zsplit<MODE, false, RB, CB, kZPD, WPE>), grid, dim3(64 * nw), 0, s, a, in, out, bt, bb);
     LSB_HIP(hipGetLastError());
     return LSB_OK;
+}
+
+// The wall-normal kernels' tiles by size.  A product loop is bound by the latency of its
+// panel and matrix loads, so what counts is the loads in flight on a CU: many pencils per
+// wave while there are blocks enough to fill the chip (kZWide pencils), one row block per
+// wave where there are few (kZFew).  Every shape sums in the same order: the same bits.
+constexpr long kZWide = 1024 * 64, kZFew = 512 * 32;
+static int zrow_blocks(const ZSplitOp& op, bool allow_xrow) {
+    return allow_xrow && (op.n & 1) && op.me > 16 && op.me % 16 == 1 ? op.me / 16 : (op.me + 15) / 16;
+}
+
+template <int MODE>
+static int launch_zs(const ZArgs& a, const ZSplitOp& op, const FieldList<double>& in, const FieldList<double>& out,
+                     const FieldList<double>& bt, const FieldList<double>& bb, int nf, hipStream_t s) {
+    if constexpr (MODE == ZM_PLAIN || MODE == ZM_AUXSUB) {
+        // d/dz, us per step (two launches of three fields) against 3 x 2 tiles: 2 x 4 tiles
+        // save 32 at 512x193x256, 33 at 256x129x128, 25 at 240x114x120 and 11 at
+        // 256x65x128 but cost 5 at 192x97x96; 1 x 2 tiles save 15 at 96x129x48 and 8 at
+        // 64x65x32 but cost 25 at 256x129x128
+        const long pencils = a.P * nf;
+        if (pencils >= kZWide) return launch_zs_shape<MODE, 2, 4, 2>(a, op, in, out, bt, bb, nf, s);
+        if (pencils < kZFew) return launch_zs_shape<MODE, 1, 2, 4>(a, op, in, out, bt, bb, nf, s);
+    }
+    // two input fields or a wider epilogue: two row blocks per wave keep three waves per SIMD
+    constexpr int RB = (MODE == ZM_PRESSDIV || MODE == ZM_PROJ) ? 2 : kZSRB;
+    return launch_zs_shape<MODE, RB, kZSCB, 3>(a, op, in, out, bt, bb, nf, s);
 }
 
 // the split kernels address a field with 32-bit element offsets
@@ -1159,8 +1184,12 @@ k_zhelm(ZArgs a, FieldList<double> fld, FieldList<double> bct, FieldList<double>
     }
 }
 // two row blocks x two column blocks per wave set (measured against 1-3 x 1-2: the
-// 49 KB LDS tile per block leaves room for three blocks per CU)
-constexpr int kZHRB = 2, kZHCB = 2;
+// 49 KB LDS tile per block leaves room for three blocks per CU); one row block per wave up
+// to 4 row blocks (n <= 128), where the smaller tiles leave room for more waves: three
+// fields of 256x129x128 124 -> 87 us, 240x114x120 90 -> 70, 192x97x96 50 -> 38,
+// 64x65x32 16 -> 10.5, but 966 -> 1135 at 512x193x256 x 4 (the panel passes the L1 once
+// per wave)
+constexpr int kZHRB = 2, kZHCB = 2, kZHSmall = 4;
 
 // The velocity solves of the mixed form: with s = k^2 + sigma much larger than every
 // |lam| (sigma = 1/(nu dt bdfv)),
@@ -1426,7 +1455,9 @@ k_zhelm32(ZArgs a, FieldList<double> fld, FieldList<double> bct, FieldList<doubl
     }
 }
 // two row blocks x three column blocks per wave set (measured against 2-4 x 2-3 on the
-// 512 x 193 x 256 step: 2 x 3 fastest; its 37 KB FP32 tile leaves room for four blocks per CU)
+// 512 x 193 x 256 step: 2 x 3 fastest; its 37 KB FP32 tile leaves room for four blocks per
+// CU).  Up to 4 row blocks: 2 x 2 tiles (us per step: -7 at 256x129x128, -4 at 192x97x96,
+// -3 at 256x65x128), 1 x 2 with few pencils (-20 at 96x129x48, -13 at 64x65x32)
 constexpr int kZH32RB = 2, kZH32CB = 3;
 
 // The pressure step of navierstokes.f90:1411-1488 for a block's 16 CB pencils in
@@ -1458,8 +1489,8 @@ struct ZPressArgs {
     double dt, bdfv;
 };
 
-template <int RB, int CB, int PD, bool XR>
-__global__ void __launch_bounds__(64 * kZMaxWaves) __attribute__((amdgpu_waves_per_eu(3)))
+template <int RB, int CB, int PD, bool XR, int WPE>
+__global__ void __launch_bounds__(64 * kZMaxWaves) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_zpress(ZPressArgs a) {
     extern __shared__ double T[];  // nzp rows x W pencils
     constexpr int W = 16 * CB;
@@ -1892,7 +1923,21 @@ k_zpress(ZPressArgs a) {
         }
     }
 }
-constexpr int kZPRB = 2, kZPCB = 2;
+// two row blocks x two column blocks per wave; up to 4 row blocks (n <= 129) one row block
+// per wave (us per step: -15 at 256x129x128, -16 at 240x114x120, -14 at 256x65x128), with
+// one column block below kZPFew pencils (-30 against -27 at 192x97x96, -21 against -16 at
+// 64x65x32, but -10 against -15 at 240x114x120)
+constexpr int kZPRB = 2, kZPCB = 2, kZPSmall = 4;
+constexpr long kZPFew = 640 * 32;
+template <int RB, int CB, int WPE>
+static void launch_zpress(const ZPressArgs& a, int nrb, hipStream_t s) {
+    const dim3 grid((unsigned)((a.P + 16 * CB - 1) / (16 * CB))), blk(64 * ((nrb + RB - 1) / RB));
+    const size_t lds = (size_t)a.nD * 16 * CB * sizeof(double);
+    if (a.xrow >= 0)
+        hipLaunchKernelGGL((k_zpress<RB, CB, kZPD, true, WPE>), grid, blk, lds, s, a);
+    else
+        hipLaunchKernelGGL((k_zpress<RB, CB, kZPD, false, WPE>), grid, blk, lds, s, a);
+}
 
 // flops of one split contraction: two me x me products per column
 static double zsplit_flops(const ZSplitOp& op, double cols) { return 4.0 * op.me * (double)op.me * cols; }
@@ -2075,6 +2120,26 @@ int zsplit_setup(lsb_ctx* c, const std::vector<double>& elift) {
     return LSB_OK;
 }
 
+template <class TI, class TO, int RB, int CB, int WPE>
+static int launch_zs32(lsb_ctx* c, const ZArgs& a0, const FieldList<TI>& fi, const FieldList<TO>& fo,
+                       const FieldList<TO>& fa, bool aux, int nf, hipStream_t s) {
+    ZArgs a = a0;
+    int gy = 1, nw = 1;
+    zsplit_shape(a, c->zs_dz, true, RB, &gy, &nw);
+    const dim3 grid((unsigned)((a.P + 16 * CB - 1) / (16 * CB)), (unsigned)gy, (unsigned)nf), blk(64 * nw);
+    const bool xr = a.xrow >= 0;
+    if (aux && xr)
+        hipLaunchKernelGGL((k_zsplit_f32<TI, TO, true, true, RB, CB, kZPD, WPE>), grid, blk, 0, s, a, fi, fo, fa);
+    else if (aux)
+        hipLaunchKernelGGL((k_zsplit_f32<TI, TO, true, false, RB, CB, kZPD, WPE>), grid, blk, 0, s, a, fi, fo, fa);
+    else if (xr)
+        hipLaunchKernelGGL((k_zsplit_f32<TI, TO, false, true, RB, CB, kZPD, WPE>), grid, blk, 0, s, a, fi, fo, fa);
+    else
+        hipLaunchKernelGGL((k_zsplit_f32<TI, TO, false, false, RB, CB, kZPD, WPE>), grid, blk, 0, s, a, fi, fo, fa);
+    LSB_HIP(hipGetLastError());
+    return LSB_OK;
+}
+
 template <class TI, class TO>
 int zcontract_f32(lsb_ctx* c, const double* M, int ldm, int nout, int nin, const TI* const* in, TO* const* out,
                   int nf, hipStream_t s, long P, const TO* const* aux) {
@@ -2098,22 +2163,19 @@ int zcontract_f32(lsb_ctx* c, const double* M, int ldm, int nout, int nin, const
     const double bytes = (double)a.P * nf * (nin * sizeof(TI) + nout * sizeof(TO) * (aux ? 2 : 1));
     int tok = -1;
     if (M == c->d_mdz && zs_fits(c->zs_dz, a.P) && nout == c->nzp && nin == c->nzp) {
-        int gy = 1, nw = 1;
-        zsplit_shape(a, c->zs_dz, true, kZSRB32, &gy, &nw);
-        dim3 grid((unsigned)((a.P + 16 * kZSCB32 - 1) / (16 * kZSCB32)), (unsigned)gy, (unsigned)nf);
         prof_mark_begin(c, PC_Z, s, &tok, zsplit_flops(c->zs_dz, (double)a.P) * nf, bytes);
-        const bool xr = a.xrow >= 0;
-        if (aux && xr)
-            hipLaunchKernelGGL((k_zsplit_f32<TI, TO, true, true>), grid, dim3(64 * nw), 0, s, a, fi, fo, fa);
-        else if (aux)
-            hipLaunchKernelGGL((k_zsplit_f32<TI, TO, true, false>), grid, dim3(64 * nw), 0, s, a, fi, fo, fa);
-        else if (xr)
-            hipLaunchKernelGGL((k_zsplit_f32<TI, TO, false, true>), grid, dim3(64 * nw), 0, s, a, fi, fo, fa);
+        // up to 4 row blocks (n <= 129), us per step against 3 x 4 tiles: 2 x 4 save 14 at
+        // 256x129x128, 4 at 240x114x120; 1 x 2 with fewer pencils 16 at 192x97x96, 17 at
+        // 96x129x48, 13 at 64x65x32 (and cost 11 at 256x129x128); 2 x 4 cost 42 at 512x193x256
+        int rc;
+        if (zrow_blocks(c->zs_dz, true) > kZHSmall)
+            rc = launch_zs32<TI, TO, kZSRB32, kZSCB32, 2>(c, a, fi, fo, fa, aux != nullptr, nf, s);
+        else if (a.P * nf >= kZWide)
+            rc = launch_zs32<TI, TO, 2, 4, 3>(c, a, fi, fo, fa, aux != nullptr, nf, s);
         else
-            hipLaunchKernelGGL((k_zsplit_f32<TI, TO, false, false>), grid, dim3(64 * nw), 0, s, a, fi, fo, fa);
+            rc = launch_zs32<TI, TO, 1, 2, 4>(c, a, fi, fo, fa, aux != nullptr, nf, s);
         prof_mark_end(c, tok, s);
-        LSB_HIP(hipGetLastError());
-        return LSB_OK;
+        return rc;
     }
     a.xrow = (nout > 16 && nout % 16 == 1) ? nout - 1 : -1;
     const int nrb = (a.xrow >= 0) ? nout / 16 : (nout + 15) / 16;
@@ -2323,18 +2385,35 @@ int zpress_step(lsb_ctx* c, double* u, double* v, const double* w, double* wout,
     a.bdfv = bdfv;
     const int nrbD = (a.xrow >= 0) ? D.me / 16 : (D.me + 15) / 16;
     const int nrbH = (H1.me + 15) / 16;
-    const int nw = (std::max(nrbD, nrbH) + kZPRB - 1) / kZPRB;
-    if (nw > kZMaxWaves) return LSB_E_UNSUPPORTED;
-    dim3 grid((unsigned)((P + 16 * kZPCB - 1) / (16 * kZPCB)));
+    const int nrb = std::max(nrbD, nrbH);
+    if (nrb > kZPRB * kZMaxWaves) return LSB_E_UNSUPPORTED;
     int tok = -1;
     // four split contractions per pencil; reads u, v, w, u, v; writes w_new, p, u, v
     prof_mark_begin(c, PC_HELM, s, &tok, 2.0 * (zsplit_flops(D, (double)P) + zsplit_flops(H1, (double)P)),
                     9.0 * c->nzp * (double)P * sizeof(double));
-    if (a.xrow >= 0)
-        hipLaunchKernelGGL((k_zpress<kZPRB, kZPCB, kZPD, true>), grid, dim3(64 * nw), lds, s, a);
+    if (nrb <= kZPSmall && P < kZPFew)
+        launch_zpress<1, 1, 4>(a, nrb, s);
+    else if (nrb <= kZPSmall)
+        launch_zpress<1, 2, 3>(a, nrb, s);
     else
-        hipLaunchKernelGGL((k_zpress<kZPRB, kZPCB, kZPD, false>), grid, dim3(64 * nw), lds, s, a);
+        launch_zpress<kZPRB, kZPCB, 3>(a, nrb, s);
     prof_mark_end(c, tok, s);
+    LSB_HIP(hipGetLastError());
+    return LSB_OK;
+}
+
+template <int RB, int CB, int PD, int WPE>
+static int launch_zhelm32(lsb_ctx* c, const ZArgs& a, const FieldList<double>& fr, const FieldList<double>& bt,
+                          const FieldList<double>& bb, int nf, hipStream_t s) {
+    ZArgs b = a;
+    int gy = 1, nw = 1;
+    zsplit_shape(b, c->zs_h1, false, RB, &gy, &nw);
+    b.M32b = c->zs_h2.d_m32;
+    b.q32b = (long)c->zs_h2.qoff;
+    b.eel = c->d_helm_s + 5 * c->nzm;
+    dim3 grid((unsigned)((a.P + 16 * CB - 1) / (16 * CB)), 1, (unsigned)nf);
+    hipLaunchKernelGGL((k_zhelm32<RB, CB, PD, WPE>), grid, dim3(64 * nw), (size_t)c->nzm * 16 * CB * sizeof(float), s,
+                       b, fr, bt, bb);
     LSB_HIP(hipGetLastError());
     return LSB_OK;
 }
@@ -2397,26 +2476,29 @@ int helmholtz(lsb_ctx* c, double* const* rhs, const double* const* bc_top, const
             // s c(lam) <= max|lam| / sigma <= 1/16 scales the FP32 rounding
             double lmax = 0.0;
             for (int k = 0; k < nzm; ++k) lmax = std::max(lmax, std::fabs(c->diag[k]));
-            int gy32 = 1, nw32 = 1;
-            ZArgs b = a;
-            zsplit_shape(b, c->zs_h1, false, kZH32RB, &gy32, &nw32);
-            b.M32b = c->zs_h2.d_m32;
-            b.q32b = (long)c->zs_h2.qoff;
-            b.eel = c->d_helm_s + 5 * nzm;
+            const int nrb = zrow_blocks(c->zs_h1, false);
             const size_t lds32 = (size_t)nzm * 16 * kZH32CB * sizeof(float);
-            if (sigma >= 16.0 * lmax && gy32 == 1 && lds32 <= 64 * 1024) {
+            if (sigma >= 16.0 * lmax && nrb <= kZH32RB * kZMaxWaves && lds32 <= 64 * 1024) {
                 // profiled with the FP32 contractions (its projections run on the FP32 matrix cores)
                 prof_mark_begin(c, PC_Z, s, &tok, hflops, bytes);
-                dim3 grid32((unsigned)((a.P + 16 * kZH32CB - 1) / (16 * kZH32CB)), 1, (unsigned)nf);
-                hipLaunchKernelGGL((k_zhelm32<kZH32RB, kZH32CB, 3, 2>), grid32, dim3(64 * nw32), lds32, s, b, fr,
-                                   bt, bb);
+                int rc;
+                if (nrb <= kZHSmall && a.P * nf < kZFew)
+                    rc = launch_zhelm32<1, 2, 3, 4>(c, a, fr, bt, bb, nf, s);
+                else if (nrb <= kZHSmall)
+                    rc = launch_zhelm32<2, 2, 3, 3>(c, a, fr, bt, bb, nf, s);
+                else
+                    rc = launch_zhelm32<kZH32RB, kZH32CB, 3, 2>(c, a, fr, bt, bb, nf, s);
                 prof_mark_end(c, tok, s);
-                LSB_HIP(hipGetLastError());
-                return LSB_OK;
+                return rc;
             }
         }
         prof_mark_begin(c, PC_HELM, s, &tok, hflops, bytes);
-        if (ok) hipLaunchKernelGGL((k_zhelm<kZHRB, kZHCB, 3, 3>), grid, dim3(64 * nw), lds, s, a, fr, bt, bb);
+        if (ok && zrow_blocks(c->zs_h1, false) <= kZHSmall) {
+            zsplit_shape(a, c->zs_h1, false, 1, &gy, &nw);
+            hipLaunchKernelGGL((k_zhelm<1, kZHCB, 2, 4>), grid, dim3(64 * nw), lds, s, a, fr, bt, bb);
+        } else if (ok) {
+            hipLaunchKernelGGL((k_zhelm<kZHRB, kZHCB, 3, 3>), grid, dim3(64 * nw), lds, s, a, fr, bt, bb);
+        }
         if (ok) {
             prof_mark_end(c, tok, s);
             LSB_HIP(hipGetLastError());
