@@ -300,9 +300,9 @@ extern "C" int lsb_destroy(lsb_ctx* c) {
     for (double* p : ds)
         if (p) (void)hipFree(p);
     if (c->d_walls) (void)hipFree(c->d_walls);
-    for (double* p : {c->zs_dz.d_m, c->zs_h1.d_m, c->zs_h2.d_m, c->d_helm_s})
+    for (double* p : {c->zs_dz.d_m, c->zs_h1.d_m, c->zs_h2.d_m, c->zs_d2.d_m, c->d_helm_s})
         if (p) (void)hipFree(p);
-    for (float* p : {c->zs_dz.d_m32, c->zs_h1.d_m32, c->zs_h2.d_m32})
+    for (float* p : {c->zs_dz.d_m32, c->zs_h1.d_m32, c->zs_h2.d_m32, c->zs_d2.d_m32})
         if (p) (void)hipFree(p);
     for (void* p : c->stage)
         if (p) (void)hipFree(p);

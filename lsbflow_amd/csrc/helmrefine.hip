@@ -11,12 +11,15 @@
 //   LSB_HELM_SPLIT32 the mixed form's velocity solve (zops.hip k_zhelm32): the FP64
 //                   leading term -rhs/(k^2 + sigma) and the FP32 projections of the
 //                   correction, used when sigma >= 16 max|lambda| (else the FP64 solve).
-// The mode values, the FP64 operator and the residual live in the context's staging
-// slots 20-22 (no other entry point uses them).
+// FP32 and REFINE run as one kernel on a grid symmetric about the mid-plane (zops.hip
+// k_zrefine).  The separate kernels here serve the other grids; their mode values, FP64
+// operator and residual live in the context's staging slots 20-22 (no other entry point
+// uses them).
 
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
 #include <vector>
 
 #include "lsb_internal.h"
@@ -107,6 +110,19 @@ int helmholtz_precision(lsb_ctx* c, double* rhs, int nf, double sigma, int mode,
         set_error("solve_helmholtz_mixed: mode must be LSB_HELM_FP64, LSB_HELM_FP32, LSB_HELM_REFINE or "
                   "LSB_HELM_SPLIT32");
         return LSB_E_ARG;
+    }
+    // everything between right-hand side and solution in LDS where the grid allows it
+    // (LSB_NO_ZREFINE=1, for tests: the separate kernels below)
+    const char* off = std::getenv("LSB_NO_ZREFINE");
+    if (!(off && off[0] == '1')) {
+        int rc = LSB_OK;
+        for (int f0 = 0; f0 < nf && rc == LSB_OK; f0 += kMaxFields) {
+            const int nb = std::min(kMaxFields, nf - f0);
+            double* r[kMaxFields];
+            for (int q = 0; q < nb; ++q) r[q] = rhs + (size_t)(f0 + q) * c->nspec;
+            rc = zrefine(c, r, nb, sigma, mode == LSB_HELM_REFINE, s);
+        }
+        if (rc != LSB_E_UNSUPPORTED) return rc;
     }
     const int nzm = c->nzm, nzp = c->nzp;
     const long P = (long)c->plane_s;

@@ -171,8 +171,9 @@ struct lsb_ctx {
     int nwalls = 0;
     // parity-split forms of dfdz (d_mdz) and of the two Helmholtz projections, with
     // the eigenvalues and Einv-lifting data in parity-ordered mode rows (d_helm_s:
-    // nzm, then 4*nzm); not built (ok = false) on a grid without the symmetry
-    lsb::ZSplitOp zs_dz, zs_h1, zs_h2;
+    // nzm, then 4*nzm), and of the interior D2; not built (ok = false) on a grid without
+    // the symmetry
+    lsb::ZSplitOp zs_dz, zs_h1, zs_h2, zs_d2;
     double* d_helm_s = nullptr;
     float* d_mdz32 = nullptr;
     float* d_smat32 = nullptr;
@@ -435,6 +436,10 @@ int zcontract_ex(lsb_ctx* c, const double* M, int ldm, int nout, int nin, const 
 // sigma dominates the eigenvalues; otherwise the FP64 projections
 int helmholtz(lsb_ctx* c, double* const* rhs, const double* const* bc_top,
               const double* const* bc_bot, int nf, double sigma, hipStream_t s, bool split32 = false);
+
+// the solve with FP32 projections, refine: and one FP64 refinement, of nf fields in place;
+// LSB_E_UNSUPPORTED when the one-kernel form does not apply
+int zrefine(lsb_ctx* c, double* const* rhs, int nf, double sigma, bool refine, hipStream_t s);
 
 // spectral pointwise (spectral.hip)
 int sp_dfdx(lsb_ctx* c, const double* in, double* out, hipStream_t s);

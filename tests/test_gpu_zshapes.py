@@ -14,6 +14,7 @@ import pytest
 import lsbflow_amd as L
 from lsbflow_amd.core import Config, Context, setup_case
 from tests.conftest import rel_l2
+from tests.test_gpu_helmholtz_c3 import Hip, c3_rhs, solve_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -66,3 +67,24 @@ def test_step_against_unfused(nx, ny, nz, monkeypatch):
     print(f"{nx}x{nz + 1}x{ny}: {errs} mixed {mixed}", flush=True)
     assert max(errs[k] for k in ("uf", "vf", "wf")) < 1e-10 and errs["pf"] < 1e-7
     assert max(mixed.values()) < 1e-6
+
+
+@pytest.mark.parametrize("nx,ny", HORIZ[:2] + [(162, 108)])
+@pytest.mark.parametrize("nz", [16, 64, 127, 129, 170, 172, 192])
+@pytest.mark.parametrize("sigma", [0.0, 2.0e5])
+def test_fp32_and_refined_solve(nx, ny, nz, sigma, monkeypatch):
+    """The one-kernel solves against the FP64 solution: FP32's rounding times the solve's
+    conditioning (the separate kernels' error up to the order of its sums), and after the
+    refinement that error times itself, at least four digits below."""
+    hip = Hip()
+    with setup_case(L.cases.CASES["c2_dyn_les"].with_(nx=nx, ny=ny, nz=nz)) as ctx:
+        rhs = c3_rhs(nz + 1, nx * ny, 2).reshape(2, nz + 1, ny, nx)
+        u64 = solve_dev(ctx, hip, rhs, sigma, 0)
+        u32, ur = (solve_dev(ctx, hip, rhs, sigma, m) for m in (1, 2))
+        monkeypatch.setenv("LSB_NO_ZREFINE", "1")
+        s32, sr = (solve_dev(ctx, hip, rhs, sigma, m) for m in (1, 2))
+    e = [rel_l2(x, u64) for x in (u32, ur, s32, sr)]
+    print(f"{nx}x{nz + 1}x{ny} sigma {sigma}: FP32 {e[0]:.1e} refined {e[1]:.1e}; separate {e[2]:.1e} {e[3]:.1e}",
+          flush=True)
+    assert np.all(ur[:, 0] == 0.0) and np.all(ur[:, nz] == 0.0) and np.all(u32[:, nz] == 0.0)
+    assert e[0] < 4.0 * e[2] and e[1] < 4.0 * max(e[3], 1e-15)
