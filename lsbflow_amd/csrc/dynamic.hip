@@ -1,10 +1,11 @@
-// Dynamic Smagorinsky model of the mixed form (sgsterm.f90:123-280) and the plane means of
-// the plane-averaged coefficient (both forms).
+// Dynamic Smagorinsky model of the step (sgsterm.f90:123-280) and the plane means of the
+// plane-averaged coefficient.  HBM-bound: the stages are passes over 34, 23 and 21 fields
+// around the test filter's 42.
 //
-// Mixed form: every work field is stored in FP32 and every expression is evaluated in FP64
-// registers.  The fields hold perturbation quantities only; the base flow U = (ubar(z), 0, 0)
-// enters the kernels as FP64 profiles, so no FP32 field carries an O(1) part that later
-// cancels:
+// The work fields are stored in FP32 in the mixed form and in FP64 otherwise; every
+// expression is evaluated in FP64 registers.  The fields hold perturbation quantities only;
+// the base flow U = (ubar(z), 0, 0) enters the kernels as FP64 profiles, so no FP32 field
+// carries an O(1) part that later cancels:
 //   stage 1  from u', g' (perturbation velocity and gradient): the advective term, the
 //            perturbation products p_lm = u_l u_m - U_l U_m, the perturbation strain
 //            S'_lm = (g'_lm + g'_ml)/2, |S| and L1_lm = delta^2 |S| S_lm of the full strain;
@@ -47,23 +48,24 @@ dim3 row_grid(const DDims& d) {
     return dim3(gx, (unsigned)(rows < 65535 ? rows : 65535));
 }
 
-// FP32 field element by byte offset: with a 32-bit offset the loads and stores take the
+// field element by byte offset: with a 32-bit offset the loads and stores take the
 // scalar-base + vector-offset form (no 64-bit address arithmetic per field)
-template <class Off>
-__device__ __forceinline__ float ldf(const float* p, Off bo) {
-    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + bo);
+template <class T, class Off>
+__device__ __forceinline__ T ldf(const T* p, Off bo) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + bo);
 }
-template <class Off>
-__device__ __forceinline__ void stf(float* p, Off bo, float v) {
-    *reinterpret_cast<float*>(reinterpret_cast<char*>(p) + bo) = v;
+template <class T, class Off>
+__device__ __forceinline__ void stf(T* p, Off bo, T v) {
+    *reinterpret_cast<T*>(reinterpret_cast<char*>(p) + bo) = v;
 }
 
 }  // namespace
 
 // stage 1 at one point of plane k (column i) from u' and g'; out: nlt (3), p (6), |S|,
 // S' (6), L1 (6) in that order
-__device__ __forceinline__ void dynm_stage1_math(const DynMixArgs& a, int k, int i, const double (&up)[3],
-                                                 const double (&g)[3][3], float (&out)[22]) {
+template <class T>
+__device__ __forceinline__ void dynm_stage1_math(const DynMixArgs<T>& a, int k, int i, const double (&up)[3],
+                                                 const double (&g)[3][3], T (&out)[22]) {
     const double U = a.ubar[k];
     double u[3];
     u[0] = up[0] + U;
@@ -78,15 +80,15 @@ __device__ __forceinline__ void dynm_stage1_math(const DynMixArgs& a, int k, int
 #pragma unroll
         for (int m = 0; m < 3; ++m) s = s - 0.5 * u[m] * ((l == 0 && m == 2) ? g02 : g[l][m]);
         if (a.lam) s = s - lam * up[l];  // lambda (target - u): target = ubar for u, 0 for v, w
-        out[l] = (float)s;
+        out[l] = (T)s;
     }
     // perturbation products: u_l u_m - U_l U_m (only U_0 = ubar is nonzero)
-    out[3] = (float)(up[0] * (u[0] + U));
-    out[4] = (float)(up[1] * u[0]);
-    out[5] = (float)(up[2] * u[0]);
-    out[6] = (float)(up[1] * up[1]);
-    out[7] = (float)(up[2] * up[1]);
-    out[8] = (float)(up[2] * up[2]);
+    out[3] = (T)(up[0] * (u[0] + U));
+    out[4] = (T)(up[1] * u[0]);
+    out[5] = (T)(up[2] * u[0]);
+    out[6] = (T)(up[1] * up[1]);
+    out[7] = (T)(up[2] * up[1]);
+    out[8] = (T)(up[2] * up[2]);
     // strain of the perturbation and of the full field
     double sp[6], sn = 0.0;
 #pragma unroll
@@ -101,26 +103,27 @@ __device__ __forceinline__ void dynm_stage1_math(const DynMixArgs& a, int k, int
     }
     sn = sqrt(sn);
     const double dl = a.delta[k];
-    out[9] = (float)sn;
+    out[9] = (T)sn;
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
-        out[10 + q] = (float)sp[q];
-        out[16 + q] = (float)(dl * dl * sn * sf[q]);
+        out[10 + q] = (T)sp[q];
+        out[16 + q] = (T)(dl * dl * sn * sf[q]);
     }
 }
 
-__device__ __forceinline__ float* dynm_stage1_dst(const DynMixArgs& a, int n) {
+template <class T>
+__device__ __forceinline__ T* dynm_stage1_dst(const DynMixArgs<T>& a, int n) {
     return n < 3 ? a.nlt[n] : n < 9 ? a.p[n - 3] : n == 9 ? a.snorm : n < 16 ? a.sp[n - 10] : a.l1[n - 16];
 }
 
-template <class Off>
-__global__ void __launch_bounds__(256) k_dynm_stage1(DDims d, DynMixArgs a) {
+template <class T, class Off>
+__global__ void __launch_bounds__(256) k_dynm_stage1(DDims d, DynMixArgs<T> a) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= d.nx) return;
     const int nrows = d.ny * d.nzp;
     for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
         const int k = row / d.ny;
-        const Off o = ((Off)row * (Off)d.nxpp + (Off)i) * (Off)sizeof(float);
+        const Off o = ((Off)row * (Off)d.nxpp + (Off)i) * (Off)sizeof(T);
         double up[3], g[3][3];
 #pragma unroll
         for (int l = 0; l < 3; ++l) up[l] = (double)ldf(a.ui[l], o);
@@ -128,7 +131,7 @@ __global__ void __launch_bounds__(256) k_dynm_stage1(DDims d, DynMixArgs a) {
         for (int l = 0; l < 3; ++l)
 #pragma unroll
             for (int m = 0; m < 3; ++m) g[l][m] = (double)ldf(a.g[l + 3 * m], o);
-        float out[22];
+        T out[22];
         dynm_stage1_math(a, k, i, up, g, out);
 #pragma unroll
         for (int n = 0; n < 22; ++n) stf(dynm_stage1_dst(a, n), o, out[n]);
@@ -137,7 +140,7 @@ __global__ void __launch_bounds__(256) k_dynm_stage1(DDims d, DynMixArgs a) {
 
 // The same with two adjacent x points per thread: 8-byte loads and stores (nx and nxpp
 // even, so every pair is 8-byte aligned), the per-point expressions unchanged.
-__global__ void __launch_bounds__(256) k_dynm_stage1x2(DDims d, DynMixArgs a) {
+__global__ void __launch_bounds__(256) k_dynm_stage1x2(DDims d, DynMixArgs<float> a) {
     const int i = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= d.nx) return;
     const int nrows = d.ny * d.nzp;
@@ -174,8 +177,9 @@ __global__ void __launch_bounds__(256) k_dynm_stage1x2(DDims d, DynMixArgs a) {
 
 // stage 2 at one point of plane k from its 21 filtered values x: S' (6), L1 (6), u' (3),
 // p (6); returns M:L and M:M
-__device__ __forceinline__ void dynm_stage2_math(const DynMixArgs& a, int nzp, int k, const double (&x)[21],
-                                                 float& num_o, float& den_o) {
+template <class T>
+__device__ __forceinline__ void dynm_stage2_math(const DynMixArgs<T>& a, int nzp, int k, const double (&x)[21],
+                                                 T& num_o, T& den_o) {
     const double Ub = a.base[k];
     const double SUh = a.base[nzp + k];
     const double LU = a.base[2 * nzp + k];
@@ -203,26 +207,27 @@ __device__ __forceinline__ void dynm_stage2_math(const DynMixArgs& a, int nzp, i
         num = num + w * mij * lij;
         den = den + w * mij * mij;
     }
-    num_o = (float)num;
-    den_o = (float)den;
+    num_o = (T)num;
+    den_o = (T)den;
 }
 
-__device__ __forceinline__ const float* dynm_stage2_src(const DynMixArgs& a, int n) {
+template <class T>
+__device__ __forceinline__ const T* dynm_stage2_src(const DynMixArgs<T>& a, int n) {
     return n < 6 ? a.sph[n] : n < 12 ? a.l1h[n - 6] : n < 15 ? a.uh[n - 12] : a.ph[n - 15];
 }
 
-template <class Off>
-__global__ void __launch_bounds__(256) k_dynm_stage2(DDims d, DynMixArgs a) {
+template <class T, class Off>
+__global__ void __launch_bounds__(256) k_dynm_stage2(DDims d, DynMixArgs<T> a) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= d.nx) return;
     const int nrows = d.ny * d.nzp;
     for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
         const int k = row / d.ny;
-        const Off o = ((Off)row * (Off)d.nxpp + (Off)i) * (Off)sizeof(float);
+        const Off o = ((Off)row * (Off)d.nxpp + (Off)i) * (Off)sizeof(T);
         double x[21];
 #pragma unroll
         for (int n = 0; n < 21; ++n) x[n] = (double)ldf(dynm_stage2_src(a, n), o);
-        float num, den;
+        T num, den;
         dynm_stage2_math(a, d.nzp, k, x, num, den);
         stf(a.num, o, num);
         stf(a.den, o, den);
@@ -230,7 +235,7 @@ __global__ void __launch_bounds__(256) k_dynm_stage2(DDims d, DynMixArgs a) {
 }
 
 // The same with two adjacent x points per thread (8-byte loads and stores).
-__global__ void __launch_bounds__(256) k_dynm_stage2x2(DDims d, DynMixArgs a) {
+__global__ void __launch_bounds__(256) k_dynm_stage2x2(DDims d, DynMixArgs<float> a) {
     const int i = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= d.nx) return;
     const int nrows = d.ny * d.nzp;
@@ -253,8 +258,8 @@ __global__ void __launch_bounds__(256) k_dynm_stage2x2(DDims d, DynMixArgs a) {
 }
 
 // stage 3 at one point of plane k from the coefficient ratio ct = <M:L> / <M:M>
-template <class Off>
-__device__ __forceinline__ void dynm_stage3_point(const DynMixArgs& a, Off o, int k, double ct) {
+template <class T, class Off>
+__device__ __forceinline__ void dynm_stage3_point(const DynMixArgs<T>& a, Off o, int k, double ct) {
     if (ct < 0.0 || isnan(ct)) ct = 0.0;
     if (ct > 0.2 * 0.2) ct = 0.2 * 0.2;
     const double dl = a.delta[k];
@@ -264,18 +269,18 @@ __device__ __forceinline__ void dynm_stage3_point(const DynMixArgs& a, Off o, in
     for (int q = 0; q < 6; ++q) {
         const double s = (double)ldf(a.sp[q], o) + (q == 2 ? su : 0.0);
         const double tau = -2.0 * nu * s;
-        stf(a.h[q], o, (float)(0.5 * (double)ldf(a.h[q], o) + tau));  // h holds p on entry
+        stf(a.h[q], o, (T)(0.5 * (double)ldf(a.h[q], o) + tau));  // h holds p on entry
     }
 }
 
-template <class Off>
-__global__ void __launch_bounds__(256) k_dynm_stage3(DDims d, DynMixArgs a) {
+template <class T, class Off>
+__global__ void __launch_bounds__(256) k_dynm_stage3(DDims d, DynMixArgs<T> a) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= d.nx) return;
     const int nrows = d.ny * d.nzp;
     for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
         const int k = row / d.ny;
-        const Off o = ((Off)row * (Off)d.nxpp + (Off)i) * (Off)sizeof(float);
+        const Off o = ((Off)row * (Off)d.nxpp + (Off)i) * (Off)sizeof(T);
         const double ct =
             a.cplane ? a.cplane[k] / a.cplane[d.nzp + k] : (double)ldf(a.numf, o) / (double)ldf(a.denf, o);
         dynm_stage3_point(a, o, k, ct);
@@ -286,22 +291,22 @@ __global__ void __launch_bounds__(256) k_dynm_stage3(DDims d, DynMixArgs a) {
 // (a TX x R tile with periodic halos global -> registers -> LDS, the x pass into a second
 // LDS array, the y pass, the z pass over three planes in registers, the next tile's loads
 // in flight) for num and den in turn on every plane, and at each output point the two
-// averages, rounded to FP32 as stored averages would be, go into stage 3.  Same
+// averages, rounded to T as stored averages would be, go into stage 3.  Same
 // expressions and order as the filter followed by k_dynm_stage3: bit-identical to them.
-template <int R, int TX>
-__global__ void __launch_bounds__(256) k_dynm_avg3(DDims d, DynMixArgs A, const double* __restrict__ w, int KC) {
+template <class T, int R, int TX>
+__global__ void __launch_bounds__(256) k_dynm_avg3(DDims d, DynMixArgs<T> A, const double* __restrict__ w, int KC) {
     constexpr int NT = (R + 2) * (TX + 2);  // tile elements
     constexpr int NL = (NT + 255) / 256;    // tile loads per thread
     constexpr int NP = (R * TX) / 256;      // output points per thread
     static_assert((R * TX) % 256 == 0, "R * TX must be a multiple of 256");
-    __shared__ float tile[NT];
+    __shared__ T tile[NT];
     __shared__ double xs[(R + 2) * TX];
     const int ntx = (d.nx + TX - 1) / TX;
     const int i0 = (blockIdx.x % ntx) * TX;
     const int J0 = (blockIdx.x / ntx) * R;
     const int k0 = blockIdx.y * KC;
     const int k1 = min(k0 + KC, d.nzp);
-    const float* src[2] = {A.num, A.den};
+    const T* src[2] = {A.num, A.den};
     const double a = 1.0, b = 1.0;
     const double s = 2. * a + b;
     const double s2 = 2.00 * a + b;
@@ -323,11 +328,11 @@ __global__ void __launch_bounds__(256) k_dynm_avg3(DDims d, DynMixArgs A, const 
         }
         toff[m] = off;
     }
-    float pre[NL];
+    T pre[NL];
     auto load = [&](int f, int k) {
-        const float* qk = src[f] + (long)k * plane;
+        const T* qk = src[f] + (long)k * plane;
 #pragma unroll
-        for (int m = 0; m < NL; ++m) pre[m] = (toff[m] >= 0) ? qk[toff[m]] : 0.f;
+        for (int m = 0; m < NL; ++m) pre[m] = (toff[m] >= 0) ? qk[toff[m]] : (T)0;
     };
     // xy-filtered values of the tile in `pre`; then the loads of (fn, kn) (kn >= 0) in flight
     auto stage = [&](double (&y)[NP], int fn, int kn) {
@@ -340,7 +345,7 @@ __global__ void __launch_bounds__(256) k_dynm_avg3(DDims d, DynMixArgs A, const 
         if (kn >= 0) load(fn, kn);
         for (int e = threadIdx.x; e < (R + 2) * TX; e += 256) {
             const int rr = e / TX, c = e - rr * TX;
-            const float* t = tile + rr * (TX + 2) + c;
+            const T* t = tile + rr * (TX + 2) + c;
             xs[e] = fdiv(a * (double)t[0] + b * (double)t[1] + a * (double)t[2], s, is, p2);
         }
         __syncthreads();
@@ -362,8 +367,8 @@ __global__ void __launch_bounds__(256) k_dynm_avg3(DDims d, DynMixArgs A, const 
             const int r = p / TX, c = p - r * TX;
             const int j = J0 + r, i = i0 + c;
             if (j < d.ny && i < d.nx) {
-                const unsigned o = (unsigned)(((k * d.ny + j) * d.nxpp + i) * (int)sizeof(float));
-                dynm_stage3_point(A, o, k, (double)(float)vn[m] / (double)(float)vd[m]);
+                const unsigned o = (unsigned)(((k * d.ny + j) * d.nxpp + i) * (int)sizeof(T));
+                dynm_stage3_point(A, o, k, (double)(T)vn[m] / (double)(T)vd[m]);
             }
         }
     };
@@ -408,10 +413,11 @@ __global__ void __launch_bounds__(256) k_dynm_avg3(DDims d, DynMixArgs A, const 
     if (k1 == d.nzp) out(d.nzp - 1, Yc[0], Yc[1]);
 }
 
-int ph_dyn_mixed_avg3(lsb_ctx* c, const DynMixArgs& a, hipStream_t s) {
+template <class T>
+int ph_dyn_mixed_avg3(lsb_ctx* c, const DynMixArgs<T>& a, hipStream_t s) {
     const DDims d = ddims(c);
     // 32-bit element offsets; the (1, 1) weights on the device
-    if ((double)d.ny * d.nzp * d.nxpp * sizeof(float) >= 2147483648.0 || a.cplane) return LSB_E_UNSUPPORTED;
+    if ((double)d.ny * d.nzp * d.nxpp * sizeof(T) >= 2147483648.0 || a.cplane) return LSB_E_UNSUPPORTED;
     const double* w = c->d_fz + 3 * c->nzp;  // the (1, 1) interpolating weights
     constexpr int R = 4, TX = 128;
     const int ntx = (d.nx + TX - 1) / TX;
@@ -423,12 +429,15 @@ int ph_dyn_mixed_avg3(lsb_ctx* c, const DynMixArgs& a, hipStream_t s) {
     const dim3 grid((unsigned)tiles, (unsigned)((d.nzp + KC - 1) / KC));
     int tok = -1;
     // num, den read; snorm, sp (6), h (6) read; h (6) written
-    prof_mark_begin(c, PC_NL, s, &tok, 0.0, 21.0 * 4.0 * (double)d.nx * d.ny * d.nzp);
-    hipLaunchKernelGGL((k_dynm_avg3<R, TX>), grid, dim3(256), 0, s, d, a, w, KC);
+    prof_mark_begin(c, PC_NL, s, &tok, 0.0, 21.0 * sizeof(T) * (double)d.nx * d.ny * d.nzp);
+    hipLaunchKernelGGL((k_dynm_avg3<T, R, TX>), grid, dim3(256), 0, s, d, a, w, KC);
     prof_mark_end(c, tok, s);
     LSB_HIP(hipGetLastError());
     return LSB_OK;
 }
+
+template int ph_dyn_mixed_avg3<float>(lsb_ctx*, const DynMixArgs<float>&, hipStream_t);
+template int ph_dyn_mixed_avg3<double>(lsb_ctx*, const DynMixArgs<double>&, hipStream_t);
 
 // Plane means of two fields over the nx physical points of every row: B partial sums per
 // plane (one block each), then the B partials of each plane summed in a fixed order.
@@ -498,47 +507,48 @@ static bool stage1_single() {
     return e && e[0] == '1';
 }
 
-int ph_dyn_mixed(lsb_ctx* c, int stage, const DynMixArgs& a, hipStream_t s) {
+template <class T>
+int ph_dyn_mixed(lsb_ctx* c, int stage, const DynMixArgs<T>& a, hipStream_t s) {
     const DDims d = ddims(c);
     const dim3 g = row_grid(d);
     int tok = -1;
-    // FP32 fields read + written per point by each stage
+    // fields read + written per point by each stage
     const double per = (stage == 1) ? 12.0 + 22.0 : (stage == 2 ? 21.0 + 2.0 : 2.0 + 1.0 + 6.0 + 12.0);
-    prof_mark_begin(c, PC_NL, s, &tok, 0.0, per * 4.0 * (double)d.nx * d.ny * d.nzp);
-    // 32-bit byte offsets while a field is below 4 GiB
-    const bool small = (double)d.ny * d.nzp * d.nxpp * sizeof(float) < 4294967296.0;
-    switch (stage) {
-        case 1:
-            if (small && (d.nx % 2) == 0 && (d.nxpp % 2) == 0 && !stage1_single()) {
-                const dim3 g2((unsigned)((d.nx / 2 + 255) / 256), g.y);
+    prof_mark_begin(c, PC_NL, s, &tok, 0.0, per * sizeof(T) * (double)d.nx * d.ny * d.nzp);
+    // 32-bit byte offsets while a field is below 4 GiB; FP32 two points per thread (8-byte
+    // accesses; FP64 has them with one)
+    const bool small = (double)d.ny * d.nzp * d.nxpp * sizeof(T) < 4294967296.0;
+    if constexpr (sizeof(T) == 4) {
+        if (stage != 3 && small && (d.nx % 2) == 0 && (d.nxpp % 2) == 0 && !stage1_single()) {
+            const dim3 g2((unsigned)((d.nx / 2 + 255) / 256), g.y);
+            if (stage == 1)
                 hipLaunchKernelGGL(k_dynm_stage1x2, g2, dim3(256), 0, s, d, a);
-            } else if (small)
-                hipLaunchKernelGGL(k_dynm_stage1<unsigned>, g, dim3(256), 0, s, d, a);
             else
-                hipLaunchKernelGGL(k_dynm_stage1<size_t>, g, dim3(256), 0, s, d, a);
-            break;
-        case 2:
-            if (small && (d.nx % 2) == 0 && (d.nxpp % 2) == 0 && !stage1_single()) {
-                const dim3 g2((unsigned)((d.nx / 2 + 255) / 256), g.y);
                 hipLaunchKernelGGL(k_dynm_stage2x2, g2, dim3(256), 0, s, d, a);
-            } else if (small)
-                hipLaunchKernelGGL(k_dynm_stage2<unsigned>, g, dim3(256), 0, s, d, a);
-            else
-                hipLaunchKernelGGL(k_dynm_stage2<size_t>, g, dim3(256), 0, s, d, a);
-            break;
-        default:
-            if (small)
-                hipLaunchKernelGGL(k_dynm_stage3<unsigned>, g, dim3(256), 0, s, d, a);
-            else
-                hipLaunchKernelGGL(k_dynm_stage3<size_t>, g, dim3(256), 0, s, d, a);
-            break;
+            prof_mark_end(c, tok, s);
+            LSB_HIP(hipGetLastError());
+            return LSB_OK;
+        }
     }
+#define LSB_DYNM(K)                                                          \
+    if (small)                                                               \
+        hipLaunchKernelGGL((K<T, unsigned>), g, dim3(256), 0, s, d, a);      \
+    else                                                                     \
+        hipLaunchKernelGGL((K<T, size_t>), g, dim3(256), 0, s, d, a);
+    switch (stage) {
+        case 1: LSB_DYNM(k_dynm_stage1) break;
+        case 2: LSB_DYNM(k_dynm_stage2) break;
+        default: LSB_DYNM(k_dynm_stage3) break;
+    }
+#undef LSB_DYNM
     prof_mark_end(c, tok, s);
     LSB_HIP(hipGetLastError());
     return LSB_OK;
 }
+template int ph_dyn_mixed<float>(lsb_ctx*, int, const DynMixArgs<float>&, hipStream_t);
+template int ph_dyn_mixed<double>(lsb_ctx*, int, const DynMixArgs<double>&, hipStream_t);
 
-// z-filtered base profiles of the mixed dynamic model (FP64, host): U^ = filter(ubar),
+// z-filtered base profiles of the fused dynamic model (FP64, host): U^ = filter(ubar),
 // (S^U)^_02 = filter(ubarp / 2), (U^2)^ - (U^)^2.  The x-y passes leave a function of z
 // unchanged; the z pass uses the interpolating weights of interior planes (the boundary
 // planes keep their value, filters.f90:450-453).

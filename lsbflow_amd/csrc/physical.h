@@ -53,43 +53,43 @@ struct DynArgs {
     const double* denf;
     const double* cplane;  // plane means <M:L>(k), <M:M>(k) (2 nzp) instead of numf/denf, or null
     double* tau[9];
-    double* h[9];          // non-null: h = uu/2 + tau written over uu (the distinct components)
-    const double* uu[9];
-    int hsym;              // h/uu are the symmetric view (6 distinct fields)
 };
 
-// mixed-form dynamic model (dynamic.hip): FP32 fields, symmetric tensors as 6 fields
-// in the order (0,0), (1,0), (2,0), (1,1), (2,1), (2,2)
+// fused dynamic model (dynamic.hip): fields of T (float in the mixed form), symmetric tensors
+// as 6 fields in the order (0,0), (1,0), (2,0), (1,1), (2,1), (2,2)
+template <class T>
 struct DynMixArgs {
-    const float* ui[3];    // perturbation velocity
-    const float* g[9];     // perturbation gradient at l + 3m
+    const T* ui[3];    // perturbation velocity
+    const T* g[9];     // perturbation gradient at l + 3m
     const double* ubar;    // nzp
     const double* ubarp;   // nzp
     const double* delta;   // nzp (dynamic widths)
     const double* lam;     // sponge lambda(x) or null
-    float* nlt[3];         // stage 1 outputs
-    float* p[6];
-    float* sp[6];
-    float* l1[6];
-    float* snorm;
-    const float* sph[6];   // stage 2 inputs (filtered)
-    const float* l1h[6];
-    const float* uh[3];
-    const float* ph[6];
+    T* nlt[3];         // stage 1 outputs
+    T* p[6];
+    T* sp[6];
+    T* l1[6];
+    T* snorm;
+    const T* sph[6];   // stage 2 inputs (filtered)
+    const T* l1h[6];
+    const T* uh[3];
+    const T* ph[6];
     const double* base;    // 3 nzp: U^, (S^U)^_02, (U^2)^ - (U^)^2
-    float* num;
-    float* den;
-    const float* numf;     // stage 3 inputs
-    const float* denf;
+    T* num;
+    T* den;
+    const T* numf;     // stage 3 inputs
+    const T* denf;
     const double* cplane;  // or the plane means (2 nzp)
-    float* h[6];           // holds p on entry, h = p/2 + tau on exit
+    T* h[6];           // holds p on entry, h = p/2 + tau on exit
 };
 
 int ph_zero_pads(lsb_ctx* c, double* const* f, int nf, hipStream_t s);
-int ph_dyn_mixed(lsb_ctx* c, int stage, const DynMixArgs& a, hipStream_t s);
+template <class T>
+int ph_dyn_mixed(lsb_ctx* c, int stage, const DynMixArgs<T>& a, hipStream_t s);
 // the (1, 1) average of num and den and stage 3 in one pass (numf, denf not written);
 // LSB_E_UNSUPPORTED where that pass does not apply (the caller runs the two steps)
-int ph_dyn_mixed_avg3(lsb_ctx* c, const DynMixArgs& a, hipStream_t s);
+template <class T>
+int ph_dyn_mixed_avg3(lsb_ctx* c, const DynMixArgs<T>& a, hipStream_t s);
 // out[k] = mean of f0 over plane k, out[nzp + k] = mean of f1 (nx physical points per row);
 // scratch: ph_plane_mean2_scratch(c) doubles
 template <class T>

@@ -355,9 +355,7 @@ __global__ void k_dyn2(PhDims d, DynArgs a) {
     }
 }
 // stage 3 (sgsterm.f90:248-267): C = <ML>/<MM> clipped to [0, 0.04], tau = -2 C delta^2 |S| S_ij;
-// <.> the local filter (numf, denf) or the plane means (cplane).  With h set, h = uu/2 + tau is
-// written over uu instead of tau (the step's h_lm = 1/2 u_l u_m + tau_lm, navierstokes.f90:769),
-// once per distinct component.
+// <.> the local filter (numf, denf) or the plane means (cplane).
 __global__ void k_dyn3(PhDims d, DynArgs a) {
     PH_LOOP(d) {
         int i, j, k;
@@ -373,13 +371,7 @@ __global__ void k_dyn3(PhDims d, DynArgs a) {
 #pragma unroll
             for (int l = 0; l < 3; ++l) {
                 const int q = l + 3 * m;
-                const double tau = -2.0 * nu * a.sij[q][off];
-                if (a.h[q]) {
-                    if (a.hsym && l < m) continue;  // (l, m) and (m, l) share one field
-                    a.h[q][off] = 0.5 * a.uu[q][off] + tau;
-                } else if (a.tau[q]) {
-                    a.tau[q][off] = tau;
-                }
+                if (a.tau[q]) a.tau[q][off] = -2.0 * nu * a.sij[q][off];
             }
     }
 }

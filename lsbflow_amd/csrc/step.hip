@@ -80,7 +80,7 @@ struct StepState {
     double bnd00_top = 0.0, bnd00_bot = 0.0;  // (0,0) Re of the unit-amplitude bound planes
     // top_bc 2: the two difference planes, two physical scratch planes and the weight m(x)
     double *cdiff[2], *cphys[2], *cweight;
-    // mixed dynamic model: z-filtered base profiles (3 nzp) and their host copy
+    // dynamic model: z-filtered base profiles (3 nzp) and their host copy
     double* dynbase = nullptr;
     std::vector<double> dynbase_h;
 };
@@ -102,13 +102,14 @@ void step_free(lsb_ctx* c) {
         }
 }
 
-// dynamic model work fields (symmetric): snorm, 5 x 6 tensors, uihat (3), num/den and filtered (4)
+// dynamic model work fields (symmetric): snorm, 5 x 6 tensors, uihat (3), num/den and filtered
+// (4); then the two-pass filter's intermediate fields
 constexpr int kDynWork = 1 + 6 * 5 + 3 + 4;
 
 static int sgs_fields(const lsb_ctx* c) {
     if (!c->cfg.sgsflag) return 0;
     switch (c->cfg.sgsmodel) {
-        case 1: return kDynWork + 6 + 6;  // work, filter tmp (6), tau (6)
+        case 1: return kDynWork + kMaxFields;
         case 3: return 24 + 9 + 9;        // ub, ub2, uibuj, filtered; filter tmp (9); tau (9)
         default: return 0;
     }
@@ -323,16 +324,6 @@ struct TView {
     int uniq[9];
 };
 
-static TView sym_view(double* const* six) {
-    // six: (0,0),(1,0),(2,0),(1,1),(2,1),(2,2)
-    TView v{};
-    const int map[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};
-    for (int q = 0; q < 9; ++q) v.p[q] = six[map[q]];
-    v.nuniq = 6;
-    const int u[6] = {0, 1, 2, 4, 5, 8};
-    for (int q = 0; q < 6; ++q) v.uniq[q] = u[q];
-    return v;
-}
 static TView full_view(double* const* nine) {
     TView v{};
     for (int q = 0; q < 9; ++q) {
@@ -354,14 +345,15 @@ static int filt_view(lsb_ctx* c, const TView& in, const TView& out, double a, do
     return ph_filter3(c, fi, fo, in.nuniq, a, b, 1, tmp, s);
 }
 
-// sgsterm.f90:123-280 with work fields carved from `w` (physical fields).
-int sgs_dynamic(lsb_ctx* c, double* const* ui, const TView& uu, const TView& g, const TView& tau, bool sym,
-                double* w, hipStream_t s, bool fuse_h = false) {
+// sgsterm.f90:123-280 on full 9-component tensors (tier A), work fields carved from `w`
+// (physical fields).
+static int sgs_dynamic(lsb_ctx* c, double* const* ui, const TView& uu, const TView& g, const TView& tau, double* w,
+                       hipStream_t s) {
     const size_t np = c->nphys;
     auto F = [&](int i) { return w + (size_t)i * np; };
     int k = 0;
     double* snorm = F(k++);
-    const int nt = sym ? 6 : 9;
+    const int nt = 9;
     double *sij_b[9], *l1_b[9], *sijh_b[9], *l1h_b[9], *uuh_b[9];
     for (int q = 0; q < nt; ++q) sij_b[q] = F(k++);
     for (int q = 0; q < nt; ++q) l1_b[q] = F(k++);
@@ -375,11 +367,11 @@ int sgs_dynamic(lsb_ctx* c, double* const* ui, const TView& uu, const TView& g, 
     double* numf = F(k++);
     double* denf = F(k++);
     double* tmp = F(k);
-    TView sij = sym ? sym_view(sij_b) : full_view(sij_b);
-    TView l1 = sym ? sym_view(l1_b) : full_view(l1_b);
-    TView sijh = sym ? sym_view(sijh_b) : full_view(sijh_b);
-    TView l1h = sym ? sym_view(l1h_b) : full_view(l1h_b);
-    TView uuh = sym ? sym_view(uuh_b) : full_view(uuh_b);
+    TView sij = full_view(sij_b);
+    TView l1 = full_view(l1_b);
+    TView sijh = full_view(sijh_b);
+    TView l1h = full_view(l1h_b);
+    TView uuh = full_view(uuh_b);
     DynArgs a{};
     for (int q = 0; q < 9; ++q) {
         a.g[q] = g.p[q];
@@ -397,11 +389,6 @@ int sgs_dynamic(lsb_ctx* c, double* const* ui, const TView& uu, const TView& g, 
     a.den = den;
     a.numf = numf;
     a.denf = denf;
-    for (int q = 0; q < 9; ++q) {
-        a.h[q] = fuse_h ? uu.p[q] : nullptr;
-        a.uu[q] = uu.p[q];
-    }
-    a.hsym = sym ? 1 : 0;
     const double fa = c->cfg.a, fb = c->cfg.b;
     LSB_TRY(ph_dyn(c, 1, a, s));
     LSB_TRY(filt_view(c, sij, sijh, fa, fb, tmp, s));
@@ -470,7 +457,7 @@ int dyn_full(lsb_ctx* c, double* ui, double* uiuj, double* g, double* tau, doubl
         g9[q] = g + q * np;
         t9[q] = tau + q * np;
     }
-    return sgs_dynamic(c, u3, full_view(uu9), full_view(g9), full_view(t9), false, work, s);
+    return sgs_dynamic(c, u3, full_view(uu9), full_view(g9), full_view(t9), work, s);
 }
 
 int isc_full(lsb_ctx* c, double* ui, double* tau, double* work, hipStream_t s) {
@@ -479,6 +466,97 @@ int isc_full(lsb_ctx* c, double* ui, double* tau, double* work, hipStream_t s) {
     for (int l = 0; l < 3; ++l) u3[l] = ui + l * np;
     for (int q = 0; q < 9; ++q) t9[q] = tau + q * np;
     return sgs_interscale(c, u3, full_view(t9), work, s);
+}
+
+// Dynamic model of the step (sgsterm.f90:123-280), fields of T: products, strain and L1
+// (stage 1), the (a, b) test filter of S', L1, u', p, M:L and M:M (stage 2), their local
+// (1, 1) average or plane means, and h = p/2 + tau over the products (stage 3).  The work
+// fields follow each other in the SGS block.  An FP64 step at 512x193x256 takes 11.86 ms so,
+// and 12.24 with the products, strain, two averages and tau as passes of their own.
+template <class T>
+static int dyn_step(lsb_ctx* c, StepState* S, hipStream_t s) {
+    StepLayout& L = S->L;
+    auto ph = [&](int slot) { return reinterpret_cast<T*>(L.phys[slot]); };
+    auto W = [&](int i) { return reinterpret_cast<T*>(L.sgs) + (size_t)i * c->nphys; };
+    auto filter = [&](const T* const* in, T* const* out, int nf, double fa, double fb) {
+        if constexpr (sizeof(T) == 4)
+            return ph_filter3_f32(c, in, out, nf, fa, fb, s);
+        else
+            return ph_filter3(c, in, out, nf, fa, fb, 1, W(kDynWork), s);
+    };
+    DynMixArgs<T> a{};
+    for (int l = 0; l < 3; ++l) {
+        a.ui[l] = ph(P_UI0 + l);
+        a.nlt[l] = ph(P_NLT0 + l);
+        a.uh[l] = W(25 + l);
+    }
+    for (int q = 0; q < 9; ++q) a.g[q] = ph(P_G0 + q);
+    a.ubar = c->d_paral;
+    a.ubarp = c->d_paral + c->nzp;
+    a.delta = c->d_delta + c->nzp;
+    a.lam = (c->cfg.forcing == 1) ? c->d_lam : nullptr;
+    for (int q = 0; q < 6; ++q) {
+        a.p[q] = ph(P_H0 + q);
+        a.h[q] = ph(P_H0 + q);
+        a.sp[q] = W(q);
+        a.l1[q] = W(6 + q);
+        a.sph[q] = W(13 + q);
+        a.l1h[q] = W(19 + q);
+        a.ph[q] = W(28 + q);
+    }
+    a.snorm = W(12);
+    a.num = W(34);
+    a.den = W(35);
+    a.numf = W(36);
+    a.denf = W(37);
+    a.base = S->dynbase;
+    LSB_TRY(ph_dyn_mixed(c, 1, a, s));
+    {
+        const T* fi[21];
+        T* fo[21];
+        for (int q = 0; q < 6; ++q) {
+            fi[q] = a.sp[q];
+            fo[q] = W(13 + q);
+            fi[6 + q] = a.l1[q];
+            fo[6 + q] = W(19 + q);
+            fi[15 + q] = a.p[q];
+            fo[15 + q] = W(28 + q);
+        }
+        for (int l = 0; l < 3; ++l) {
+            fi[12 + l] = a.ui[l];
+            fo[12 + l] = W(25 + l);
+        }
+        LSB_TRY(filter(fi, fo, 21, c->cfg.a, c->cfg.b));
+    }
+    LSB_TRY(ph_dyn_mixed(c, 2, a, s));
+    if (c->cfg.dyn_avg) {
+        double* scr = reinterpret_cast<double*>(W(kDynWork));
+        double* cp = scr + ph_plane_mean2_scratch(c);
+        LSB_TRY(ph_plane_mean2<T>(c, a.num, a.den, scr, cp, s));
+        a.cplane = cp;
+    } else {
+        // the (1, 1) average and stage 3 in one pass; LSB_NO_DYNFUSE=1 (for tests) or
+        // fields above 2 GiB: the averages through HBM, then stage 3
+        const char* e = std::getenv("LSB_NO_DYNFUSE");
+        const int rf = (e && e[0] == '1') ? LSB_E_UNSUPPORTED : ph_dyn_mixed_avg3(c, a, s);
+        if (rf != LSB_E_UNSUPPORTED) return rf;
+        const T* fi[2] = {a.num, a.den};
+        T* fo[2] = {W(36), W(37)};
+        LSB_TRY(filter(fi, fo, 2, 1.0, 1.0));
+    }
+    return ph_dyn_mixed(c, 3, a, s);
+}
+
+// the dynamic model's z-filtered base profiles, uploaded where the base flow has changed
+static int dyn_base_ready(lsb_ctx* c, StepState* S) {
+    if (c->cfg.sgsflag != 1 || c->cfg.sgsmodel != 1) return LSB_OK;
+    std::vector<double> h;
+    dyn_base_profiles(c, h);
+    if (h == S->dynbase_h) return LSB_OK;
+    S->dynbase_h.swap(h);
+    LSB_HIP(hipMemcpyAsync(S->dynbase, S->dynbase_h.data(), S->dynbase_h.size() * sizeof(double),
+                           hipMemcpyHostToDevice, c->stream));
+    return LSB_OK;
 }
 
 // ------------------------------------------------------- nonlinear term
@@ -554,20 +632,7 @@ static int nlterm_phys(lsb_ctx* c, StepState* S, const double* const* uif, doubl
         LSB_TRY(ph_smag_factor(c, L.phys[P_G0 + 6], c->d_paral + c->nzp, c->cfg.cs, s));
         LSB_TRY(ph_nonlinear(c, NL_STATIC, a, s));
     } else if (model == 1) {
-        // products first (base flow added in place), then the dynamic model
-        a.write_base = 1;
-        LSB_TRY(ph_nonlinear(c, NL_PREP, a, s));
-        double* six[6] = {hph[0], hph[1], hph[2], hph[4], hph[5], hph[8]};
-        TView uu = sym_view(six);
-        double* gq[9];
-        for (int q = 0; q < 9; ++q) gq[q] = L.phys[P_G0 + q];
-        TView gv = full_view(gq);
-        double* tb[6];
-        for (int q = 0; q < 6; ++q) tb[q] = L.sgs + (size_t)(kDynWork + 6 + q) * c->nphys;  // after work + tmp
-        TView tau = sym_view(tb);
-        double* ui[3] = {L.phys[P_UI0], L.phys[P_UI0 + 1], L.phys[P_UI0 + 2]};
-        // h = 1/2 uu + tau written over uu by the model's last stage
-        LSB_TRY(sgs_dynamic(c, ui, uu, gv, tau, true, L.sgs, s, true));
+        LSB_TRY(dyn_step<double>(c, S, s));
     } else if (model == 3) {
         // interscale: tau from the filtered velocity, then h = 1/2 uu + tau (9 fields)
         double* ui[3] = {L.phys[P_UI0], L.phys[P_UI0 + 1], L.phys[P_UI0 + 2]};
@@ -627,77 +692,6 @@ static bool mixed_chain(const lsb_ctx* c) {
     return mixed_form(c) && !(c->cfg.sgsflag == 1 && c->cfg.sgsmodel == 3);
 }
 
-// Mixed form, dynamic model (sgsterm.f90:123-280): products, strain and L1 (stage 1), the
-// (a, b) test filter of S', L1, u', p in FP32, M:L and M:M (stage 2), their local (1, 1)
-// average or plane means, and h = p/2 + tau over the products (stage 3).  The FP32 work
-// fields follow each other in the SGS block.
-static int dyn_mixed(lsb_ctx* c, StepState* S, hipStream_t s) {
-    StepLayout& L = S->L;
-    auto ph = [&](int slot) { return reinterpret_cast<float*>(L.phys[slot]); };
-    auto W = [&](int i) { return reinterpret_cast<float*>(L.sgs) + (size_t)i * c->nphys; };
-    DynMixArgs a{};
-    for (int l = 0; l < 3; ++l) {
-        a.ui[l] = ph(P_UI0 + l);
-        a.nlt[l] = ph(P_NLT0 + l);
-        a.uh[l] = W(25 + l);
-    }
-    for (int q = 0; q < 9; ++q) a.g[q] = ph(P_G0 + q);
-    a.ubar = c->d_paral;
-    a.ubarp = c->d_paral + c->nzp;
-    a.delta = c->d_delta + c->nzp;
-    a.lam = (c->cfg.forcing == 1) ? c->d_lam : nullptr;
-    for (int q = 0; q < 6; ++q) {
-        a.p[q] = ph(P_H0 + q);
-        a.h[q] = ph(P_H0 + q);
-        a.sp[q] = W(q);
-        a.l1[q] = W(6 + q);
-        a.sph[q] = W(13 + q);
-        a.l1h[q] = W(19 + q);
-        a.ph[q] = W(28 + q);
-    }
-    a.snorm = W(12);
-    a.num = W(34);
-    a.den = W(35);
-    a.numf = W(36);
-    a.denf = W(37);
-    a.base = S->dynbase;
-    LSB_TRY(ph_dyn_mixed(c, 1, a, s));
-    {
-        const float* fi[21];
-        float* fo[21];
-        for (int q = 0; q < 6; ++q) {
-            fi[q] = a.sp[q];
-            fo[q] = W(13 + q);
-            fi[6 + q] = a.l1[q];
-            fo[6 + q] = W(19 + q);
-            fi[15 + q] = a.p[q];
-            fo[15 + q] = W(28 + q);
-        }
-        for (int l = 0; l < 3; ++l) {
-            fi[12 + l] = a.ui[l];
-            fo[12 + l] = W(25 + l);
-        }
-        LSB_TRY(ph_filter3_f32(c, fi, fo, 21, c->cfg.a, c->cfg.b, s));
-    }
-    LSB_TRY(ph_dyn_mixed(c, 2, a, s));
-    if (c->cfg.dyn_avg) {
-        double* scr = reinterpret_cast<double*>(W(38));
-        double* cp = scr + ph_plane_mean2_scratch(c);
-        LSB_TRY(ph_plane_mean2<float>(c, a.num, a.den, scr, cp, s));
-        a.cplane = cp;
-    } else {
-        // the (1, 1) average and stage 3 in one pass; LSB_NO_DYNFUSE=1 (for tests) or
-        // fields above 2 GiB: the averages through HBM, then stage 3
-        const char* e = std::getenv("LSB_NO_DYNFUSE");
-        const int rf = (e && e[0] == '1') ? LSB_E_UNSUPPORTED : ph_dyn_mixed_avg3(c, a, s);
-        if (rf != LSB_E_UNSUPPORTED) return rf;
-        const float* fi[2] = {a.num, a.den};
-        float* fo[2] = {W(36), W(37)};
-        LSB_TRY(ph_filter3_f32(c, fi, fo, 2, 1.0, 1.0, s));
-    }
-    return ph_dyn_mixed(c, 3, a, s);
-}
-
 // FP32 chain of the mixed form (sigma, static or no SGS model): the 9 + 3 inverse
 // transforms, the products and the SGS model in one pass (FP64 arithmetic on FP32
 // storage), 3 + 6 forward transforms to FP32 spectra (nltf_out and hf hold FP32).
@@ -753,7 +747,7 @@ static int nlterm_phys_mixed(lsb_ctx* c, StepState* S, const double* const* uif,
     } else if (model == 2) {
         LSB_TRY(ph_nonlinear_f32(c, NL_SIGMA, a, s));
     } else if (model == 1) {
-        LSB_TRY(dyn_mixed(c, S, s));
+        LSB_TRY(dyn_step<float>(c, S, s));
     } else {
         LSB_TRY(ph_smag_factor_f32(c, ph(P_G0 + 6), c->d_paral + c->nzp, c->cfg.cs, s));
         LSB_TRY(ph_nonlinear_f32(c, NL_STATIC, a, s));
@@ -835,6 +829,7 @@ int nlterm_dev(lsb_ctx* c, const double* const* uif, double* const* nlt, hipStre
     LSB_TRY(step_alloc(c));
     StepState* S = state_of(c);
     const bool sym = !(c->cfg.sgsflag == 1 && c->cfg.sgsmodel == 3);
+    LSB_TRY(dyn_base_ready(c, S));
     double* hf[9];
     hf_view(S, sym, hf);
     double* nltf[3] = {S->L.spec[S_NLTF0], S->L.spec[S_NLTF0 + 1], S->L.spec[S_NLTF0 + 2]};
@@ -1176,16 +1171,11 @@ int step_run(lsb_ctx* c, int nsteps, bool with_norm) {
         set_error("timestep: call lsb_state_set first");
         return LSB_E_STATE;
     }
-    if (mixed_form(c) && c->cfg.sgsflag == 1 && c->cfg.sgsmodel == 1) {
-        // the mixed dynamic model's z-filtered base profiles (the base flow may have changed)
-        dyn_base_profiles(c, S->dynbase_h);
-        LSB_HIP(hipMemcpyAsync(S->dynbase, S->dynbase_h.data(), S->dynbase_h.size() * sizeof(double),
-                               hipMemcpyHostToDevice, c->stream));
-    }
     if (c->graphs_live) {
         set_error("timestep: the context belongs to a captured ensemble; step it with lsb_ensemble_timestep");
         return LSB_E_STATE;
     }
+    LSB_TRY(dyn_base_ready(c, S));
     for (int n = 0; n < nsteps; ++n) {
         if (with_norm) {
             LSB_TRY(step_enqueue(c));
