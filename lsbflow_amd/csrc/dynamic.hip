@@ -1,6 +1,10 @@
 // Dynamic Smagorinsky model of the step (sgsterm.f90:123-280) and the plane means of the
-// plane-averaged coefficient.  HBM-bound: the stages are passes over 34, 23 and 21 fields
-// around the test filter's 42.
+// plane-averaged coefficient.  Two passes read u' and g' (12 fields): k_dynm_test (stages 1
+// and 2 with the test filter between them, 2 fields out), and k_dynm_avg3 or k_dynm_plane3
+// (the average and stage 3, with what that takes of stage 1 again; 9 fields out).  The
+// stages as passes of their own around the filter (what tests compare with) go over 34, 42,
+// 23, 4 and 21 fields: the FP64 step at 512x193x256 took 11.86 ms so and takes 8.32, the
+// mixed step at 256x129x128 1.26 and 1.00.
 //
 // The work fields are stored in FP32 in the mixed form and in FP64 otherwise; every
 // expression is evaluated in FP64 registers.  The fields hold perturbation quantities only;
@@ -61,17 +65,11 @@ __device__ __forceinline__ void stf(T* p, Off bo, T v) {
 
 }  // namespace
 
-// stage 1 at one point of plane k (column i) from u' and g'; out: nlt (3), p (6), |S|,
-// S' (6), L1 (6) in that order
+// advective term -1/2 u_m du_l/dx_m with the full gradient (g'_02 + ubarp), and the sponge
 template <class T>
-__device__ __forceinline__ void dynm_stage1_math(const DynMixArgs<T>& a, int k, int i, const double (&up)[3],
-                                                 const double (&g)[3][3], T (&out)[22]) {
-    const double U = a.ubar[k];
-    double u[3];
-    u[0] = up[0] + U;
-    u[1] = up[1];
-    u[2] = up[2];
-    // advective term -1/2 u_m du_l/dx_m with the full gradient (g'_02 + ubarp), sponge
+__device__ __forceinline__ void dynm_adv(const DynMixArgs<T>& a, int k, int i, const double (&up)[3],
+                                         const double (&g)[3][3], T (&nlt)[3]) {
+    const double u[3] = {up[0] + a.ubar[k], up[1], up[2]};
     const double g02 = g[0][2] + a.ubarp[k];
     const double lam = a.lam ? a.lam[i] : 0.0;
 #pragma unroll
@@ -80,40 +78,58 @@ __device__ __forceinline__ void dynm_stage1_math(const DynMixArgs<T>& a, int k, 
 #pragma unroll
         for (int m = 0; m < 3; ++m) s = s - 0.5 * u[m] * ((l == 0 && m == 2) ? g02 : g[l][m]);
         if (a.lam) s = s - lam * up[l];  // lambda (target - u): target = ubar for u, 0 for v, w
-        out[l] = (T)s;
+        nlt[l] = (T)s;
     }
-    // perturbation products: u_l u_m - U_l U_m (only U_0 = ubar is nonzero)
-    out[3] = (T)(up[0] * (u[0] + U));
-    out[4] = (T)(up[1] * u[0]);
-    out[5] = (T)(up[2] * u[0]);
-    out[6] = (T)(up[1] * up[1]);
-    out[7] = (T)(up[2] * up[1]);
-    out[8] = (T)(up[2] * up[2]);
-    // strain of the perturbation and of the full field
+}
+
+// perturbation products: u_l u_m - U_l U_m (only U_0 = ubar is nonzero)
+template <class T>
+__device__ __forceinline__ void dynm_products(const DynMixArgs<T>& a, int k, const double (&up)[3], T (&p)[6]) {
+    const double U = a.ubar[k];
+    const double u0 = up[0] + U;
+    p[0] = (T)(up[0] * (u0 + U));
+    p[1] = (T)(up[1] * u0);
+    p[2] = (T)(up[2] * u0);
+    p[3] = (T)(up[1] * up[1]);
+    p[4] = (T)(up[2] * up[1]);
+    p[5] = (T)(up[2] * up[2]);
+}
+
+// strain S' of the perturbation, |S| and S of the full field (sf)
+template <class T>
+__device__ __forceinline__ void dynm_strain(const DynMixArgs<T>& a, int k, const double (&g)[3][3], T (&spo)[6],
+                                            double (&sf)[6], double& sno) {
     double sp[6], sn = 0.0;
 #pragma unroll
     for (int q = 0; q < 6; ++q) sp[q] = 0.5 * (g[kL[q]][kM[q]] + g[kM[q]][kL[q]]);
     const double su = 0.5 * a.ubarp[k];  // base strain S^U_20 = S^U_02
-    double sf[6];
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
         sf[q] = sp[q] + (q == 2 ? su : 0.0);
         const double w = (kL[q] == kM[q]) ? 1.0 : 2.0;  // off-diagonals appear twice
         sn = sn + w * 2.0 * sf[q] * sf[q];
+        spo[q] = (T)sp[q];
     }
-    sn = sqrt(sn);
-    const double dl = a.delta[k];
-    out[9] = (T)sn;
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        out[10 + q] = (T)sp[q];
-        out[16 + q] = (T)(dl * dl * sn * sf[q]);
-    }
+    sno = sqrt(sn);
 }
 
 template <class T>
-__device__ __forceinline__ T* dynm_stage1_dst(const DynMixArgs<T>& a, int n) {
-    return n < 3 ? a.nlt[n] : n < 9 ? a.p[n - 3] : n == 9 ? a.snorm : n < 16 ? a.sp[n - 10] : a.l1[n - 16];
+__device__ __forceinline__ void dynm_l1(const DynMixArgs<T>& a, int k, const double (&sf)[6], double sn,
+                                        T (&l1)[6]) {
+    const double dl = a.delta[k];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) l1[q] = (T)(dl * dl * sn * sf[q]);
+}
+
+// u' and g' of a point (byte offset o)
+template <class T, class Off>
+__device__ __forceinline__ void dynm_load(const DynMixArgs<T>& a, Off o, double (&up)[3], double (&g)[3][3]) {
+#pragma unroll
+    for (int l = 0; l < 3; ++l) up[l] = (double)ldf(a.ui[l], o);
+#pragma unroll
+    for (int l = 0; l < 3; ++l)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) g[l][m] = (double)ldf(a.g[l + 3 * m], o);
 }
 
 template <class T, class Off>
@@ -124,69 +140,37 @@ __global__ void __launch_bounds__(256) k_dynm_stage1(DDims d, DynMixArgs<T> a) {
     for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
         const int k = row / d.ny;
         const Off o = ((Off)row * (Off)d.nxpp + (Off)i) * (Off)sizeof(T);
-        double up[3], g[3][3];
+        double up[3], g[3][3], sf[6], sn;
+        dynm_load(a, o, up, g);
+        T nlt[3], p[6], sp[6], l1[6];
+        dynm_adv(a, k, i, up, g, nlt);
+        dynm_products(a, k, up, p);
+        dynm_strain(a, k, g, sp, sf, sn);
+        dynm_l1(a, k, sf, sn, l1);
 #pragma unroll
-        for (int l = 0; l < 3; ++l) up[l] = (double)ldf(a.ui[l], o);
+        for (int l = 0; l < 3; ++l) stf(a.nlt[l], o, nlt[l]);
+        stf(a.snorm, o, (T)sn);
 #pragma unroll
-        for (int l = 0; l < 3; ++l)
-#pragma unroll
-            for (int m = 0; m < 3; ++m) g[l][m] = (double)ldf(a.g[l + 3 * m], o);
-        T out[22];
-        dynm_stage1_math(a, k, i, up, g, out);
-#pragma unroll
-        for (int n = 0; n < 22; ++n) stf(dynm_stage1_dst(a, n), o, out[n]);
-    }
-}
-
-// The same with two adjacent x points per thread: 8-byte loads and stores (nx and nxpp
-// even, so every pair is 8-byte aligned), the per-point expressions unchanged.
-__global__ void __launch_bounds__(256) k_dynm_stage1x2(DDims d, DynMixArgs<float> a) {
-    const int i = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= d.nx) return;
-    const int nrows = d.ny * d.nzp;
-    for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
-        const int k = row / d.ny;
-        const unsigned o = ((unsigned)row * (unsigned)d.nxpp + (unsigned)i) * (unsigned)sizeof(float);
-        auto ld2 = [&](const float* p) {
-            return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(p) + o);
-        };
-        double up[2][3], g[2][3][3];
-#pragma unroll
-        for (int l = 0; l < 3; ++l) {
-            const float2 v = ld2(a.ui[l]);
-            up[0][l] = (double)v.x;
-            up[1][l] = (double)v.y;
+        for (int q = 0; q < 6; ++q) {
+            stf(a.p[q], o, p[q]);
+            stf(a.sp[q], o, sp[q]);
+            stf(a.l1[q], o, l1[q]);
         }
-#pragma unroll
-        for (int l = 0; l < 3; ++l)
-#pragma unroll
-            for (int m = 0; m < 3; ++m) {
-                const float2 v = ld2(a.g[l + 3 * m]);
-                g[0][l][m] = (double)v.x;
-                g[1][l][m] = (double)v.y;
-            }
-        float out[2][22];
-        dynm_stage1_math(a, k, i, up[0], g[0], out[0]);
-        dynm_stage1_math(a, k, i + 1, up[1], g[1], out[1]);
-#pragma unroll
-        for (int n = 0; n < 22; ++n)
-            *reinterpret_cast<float2*>(reinterpret_cast<char*>(dynm_stage1_dst(a, n)) + o) =
-                make_float2(out[0][n], out[1][n]);
     }
 }
 
-// stage 2 at one point of plane k from its 21 filtered values x: S' (6), L1 (6), u' (3),
-// p (6); returns M:L and M:M
-template <class T>
-__device__ __forceinline__ void dynm_stage2_math(const DynMixArgs<T>& a, int nzp, int k, const double (&x)[21],
-                                                 T& num_o, T& den_o) {
+// stage 2 at one point of plane k from its 21 filtered values get(n), n: S' (6), L1 (6),
+// u' (3), p (6), each taken once, when it is needed; returns M:L and M:M
+template <class T, class Get>
+__device__ __forceinline__ void dynm_stage2_math(const DynMixArgs<T>& a, int nzp, int k, Get get, T& num_o,
+                                                 T& den_o) {
     const double Ub = a.base[k];
     const double SUh = a.base[nzp + k];
     const double LU = a.base[2 * nzp + k];
     double sh[6], snh = 0.0;
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
-        sh[q] = x[q] + (q == 2 ? SUh : 0.0);
+        sh[q] = get(q) + (q == 2 ? SUh : 0.0);
         const double w = (kL[q] == kM[q]) ? 1.0 : 2.0;
         snh = snh + w * 2.0 * sh[q] * sh[q];
     }
@@ -194,14 +178,14 @@ __device__ __forceinline__ void dynm_stage2_math(const DynMixArgs<T>& a, int nzp
     const double cd = 2.0 * a.delta[k];
     double uh[3];
 #pragma unroll
-    for (int l = 0; l < 3; ++l) uh[l] = x[12 + l];
+    for (int l = 0; l < 3; ++l) uh[l] = get(12 + l);
     const double Uh[3] = {Ub, 0.0, 0.0};
     double num = 0.0, den = 0.0;
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
         const int l = kL[q], m = kM[q];
-        const double mij = 2.0 * (x[6 + q] - cd * cd * snh * sh[q]);
-        double lij = x[15 + q] - (Uh[l] * uh[m] + uh[l] * Uh[m] + uh[l] * uh[m]);
+        const double mij = 2.0 * (get(6 + q) - cd * cd * snh * sh[q]);
+        double lij = get(15 + q) - (Uh[l] * uh[m] + uh[l] * Uh[m] + uh[l] * uh[m]);
         if (q == 0) lij = lij + LU;
         const double w = (l == m) ? 1.0 : 2.0;
         num = num + w * mij * lij;
@@ -224,36 +208,156 @@ __global__ void __launch_bounds__(256) k_dynm_stage2(DDims d, DynMixArgs<T> a) {
     for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
         const int k = row / d.ny;
         const Off o = ((Off)row * (Off)d.nxpp + (Off)i) * (Off)sizeof(T);
-        double x[21];
-#pragma unroll
-        for (int n = 0; n < 21; ++n) x[n] = (double)ldf(dynm_stage2_src(a, n), o);
         T num, den;
-        dynm_stage2_math(a, d.nzp, k, x, num, den);
+        dynm_stage2_math(a, d.nzp, k, [&](int n) { return (double)ldf(dynm_stage2_src(a, n), o); }, num, den);
         stf(a.num, o, num);
         stf(a.den, o, den);
     }
 }
 
-// The same with two adjacent x points per thread (8-byte loads and stores).
-__global__ void __launch_bounds__(256) k_dynm_stage2x2(DDims d, DynMixArgs<float> a) {
-    const int i = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= d.nx) return;
-    const int nrows = d.ny * d.nzp;
-    for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
-        const int k = row / d.ny;
-        const unsigned o = ((unsigned)row * (unsigned)d.nxpp + (unsigned)i) * (unsigned)sizeof(float);
-        double x[2][21];
+// Value of the lane before / after (whole-wave shift by one; the first / last lane gets 0).
+__device__ __forceinline__ float lane_prev(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_next(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double lane_prev(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x138, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double lane_next(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x130, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x130, 0xf, 0xf, true));
+}
+
+// M:L and M:M straight from u' and g': stage 1, the test filter of its 21 fields and
+// stage 2 in one pass.  A block owns txo <= 62 columns by R rows and slides over KC planes;
+// wave r holds row J0 - 1 + r (the first and the last are the y halo), lane t column
+// i0 - 1 + t (lanes 0 and txo + 1 are the x halo), both periodic.  Per plane: stage 1 at the
+// lane's point, the x pass with the neighbour lanes' values, one LDS store per field; then
+// on the R inner rows the y pass from LDS and the z pass, with the last plane's values
+// (zb) and the sum over the last two (za) in registers, and stage 2.  The loads of
+// the next plane are in flight meanwhile.  The 21 values are rounded to T where the separate
+// passes store them, in their expressions: the same bits.
+// 14 field passes in place of 99; bound by the vector units (some 410 instructions per point
+// and plane, 4/3 of the x phase for the halo rows) with HBM close behind.  R = 6: 8 waves
+// with up to 256 registers (42 FP64 values of the z pass each); R = 4 and R = 10 leave 168 and spill (FP64
+// step at 512x193x256: 8.36 ms against 10.6 and 13.3).  At that grid 1.07 ms in place of
+// 1.62 + 2.08 + 0.94 for stage 1, the filter and stage 2.
+template <class T, int R, bool P2>
+__global__ void __launch_bounds__(64 * (R + 2)) k_dynm_test(DDims d, DynMixArgs<T> A, const double* __restrict__ w,
+                                                            double fa, double fb, int txo, int KC) {
+    __shared__ double xs[21][R + 2][64];
+    const int lane = threadIdx.x & 63;
+    const int r = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ntx = (d.nx + txo - 1) / txo;
+    const int i0 = (blockIdx.x % ntx) * txo;
+    const int J0 = (blockIdx.x / ntx) * R;
+    const int k0 = blockIdx.y * KC;
+    const int k1 = min(k0 + KC, d.nzp);
+    // a sum a + b + a that is a power of two goes into the weights (exact)
+    const double s = 2. * fa + fb;
+    const double is = P2 ? 1.0 / s : 1.0;
+    const double wa = fa * is, wb = fb * is;
+    auto div = [&](double x) { return P2 ? x : x / s; };
+    int i = (i0 - 1 + lane) % d.nx;
+    i = (i < 0) ? i + d.nx : i;
+    int j = (J0 - 1 + r) % d.ny;
+    j = (j < 0) ? j + d.ny : j;
+    const unsigned off = ((unsigned)j * (unsigned)d.nxpp + (unsigned)i) * (unsigned)sizeof(T);
+    const size_t plane = (size_t)d.ny * d.nxpp;
+    const bool live = lane >= 1 && lane <= txo && i0 + lane - 1 < d.nx && J0 + r - 1 < d.ny;
+    T pre[12];
+    auto load = [&](int k) {
+        // scalar base + 32-bit lane offset, not 12 lane pointers (the asm keeps the widening
+        // of the offset from being hoisted out of the loop)
+        const size_t pl = (size_t)k * plane;
+        unsigned o = off;
+        asm("" : "+v"(o));
 #pragma unroll
-        for (int n = 0; n < 21; ++n) {
-            const float2 v = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(dynm_stage2_src(a, n)) + o);
-            x[0][n] = (double)v.x;
-            x[1][n] = (double)v.y;
+        for (int l = 0; l < 3; ++l) pre[l] = ldf(A.ui[l] + pl, o);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) pre[3 + q] = ldf(A.g[q] + pl, o);
+    };
+    auto put = [&](int k, T num, T den) {
+        if (live) {
+            stf(A.num + k * plane, off, num);
+            stf(A.den + k * plane, off, den);
         }
-        float num[2], den[2];
-        dynm_stage2_math(a, d.nzp, k, x[0], num[0], den[0]);
-        dynm_stage2_math(a, d.nzp, k, x[1], num[1], den[1]);
-        *reinterpret_cast<float2*>(reinterpret_cast<char*>(a.num) + o) = make_float2(num[0], num[1]);
-        *reinterpret_cast<float2*>(reinterpret_cast<char*>(a.den) + o) = make_float2(den[0], den[1]);
+    };
+    const int klast = min(k1, d.nzp - 1);
+    const int kstart = (k0 > 0) ? k0 - 1 : k0;
+    // stage 1 and the x pass of plane kk into LDS, the loads of the next plane behind them
+    auto xphase = [&](int kk) {
+        auto xpass = [&](int f, T v) {
+            xs[f][r][lane] = div(wa * (double)lane_prev(v) + wb * (double)v + wa * (double)lane_next(v));
+        };
+        double up[3], g[3][3], sf[6], sn;
+        T t6[6];
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+            up[l] = (double)pre[l];
+            xpass(12 + l, pre[l]);
+        }
+        dynm_products(A, kk, up, t6);
+#pragma unroll
+        for (int q = 0; q < 6; ++q) xpass(15 + q, t6[q]);
+#pragma unroll
+        for (int l = 0; l < 3; ++l)
+#pragma unroll
+            for (int m = 0; m < 3; ++m) g[l][m] = (double)pre[3 + l + 3 * m];
+        dynm_strain(A, kk, g, t6, sf, sn);
+#pragma unroll
+        for (int q = 0; q < 6; ++q) xpass(q, t6[q]);
+        dynm_l1(A, kk, sf, sn, t6);
+#pragma unroll
+        for (int q = 0; q < 6; ++q) xpass(6 + q, t6[q]);
+        if (kk < klast) load(kk + 1);
+        __syncthreads();
+    };
+    load(kstart);
+    if (r == 0 || r == R + 1) {  // the y halo rows
+        for (int kk = kstart; kk <= klast; ++kk) {
+            xphase(kk);
+            __syncthreads();
+        }
+        return;
+    }
+    double za[21], zb[21];
+#pragma unroll
+    for (int f = 0; f < 21; ++f) za[f] = zb[f] = 0.0;
+    for (int kk = kstart; kk <= klast; ++kk) {
+        xphase(kk);
+        // weights of plane kk - 1 (w0) and kk (w1) in the output plane kk and of kk in kk - 1
+        // (w2); a boundary plane keeps its value (weights 0, 1, 0)
+        const bool zin = kk - 1 > 0;  // the output plane kk - 1 is below nzp - 1
+        const bool end = kk == 0 || kk == d.nzp - 1;
+        const double w2 = zin ? is * w[2 * d.nzp + kk - 1] : 0.0;
+        const double w1 = end ? 1.0 : is * w[d.nzp + kk];
+        const double w0 = end ? 0.0 : is * w[kk];
+        auto yz = [&](int f) {
+            const double y = div(wa * xs[f][r - 1][lane] + wb * xs[f][r][lane] + wa * xs[f][r + 1][lane]);
+            // z = za + w2 y, za = w0 zb + w1 y in the three-address form (the two-address one
+            // costs copies of the sums on every plane)
+            const double t = w1 * y;
+            double z;
+            asm("v_fma_f64 %0, %1, %2, %3" : "=v"(z) : "s"(w2), "v"(y), "v"(za[f]));
+            asm("v_fma_f64 %0, %1, %2, %3" : "=v"(za[f]) : "s"(w0), "v"(zb[f]), "v"(t));
+            zb[f] = y;
+            if constexpr (!P2) z = zin ? z / s : z;
+            return (double)(T)z;
+        };
+        T num, den;
+        dynm_stage2_math(A, d.nzp, max(kk - 1, 0), yz, num, den);
+        if (kk > k0) put(kk - 1, num, den);
+        __syncthreads();
+    }
+    // the last plane of the grid keeps its xy-filtered value (no z pass)
+    if (k1 == d.nzp) {
+        T num, den;
+        dynm_stage2_math(A, d.nzp, d.nzp - 1, [&](int f) { return (double)(T)za[f]; }, num, den);
+        put(d.nzp - 1, num, den);
     }
 }
 
@@ -284,6 +388,49 @@ __global__ void __launch_bounds__(256) k_dynm_stage3(DDims d, DynMixArgs<T> a) {
         const double ct =
             a.cplane ? a.cplane[k] / a.cplane[d.nzp + k] : (double)ldf(a.numf, o) / (double)ldf(a.denf, o);
         dynm_stage3_point(a, o, k, ct);
+    }
+}
+
+// Stage 3 at one point from u' and g': what it takes of stage 1 (N pieces, products, |S|,
+// S') again at the point, rounded to T where the separate stages store it.
+template <class T>
+__device__ __forceinline__ void dynm_tau_point(const DynMixArgs<T>& a, size_t pl, unsigned o, int k, int i,
+                                               double ct) {
+    if (ct < 0.0 || isnan(ct)) ct = 0.0;
+    if (ct > 0.2 * 0.2) ct = 0.2 * 0.2;
+    double up[3], g[3][3], sf[6], sn;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) up[l] = (double)ldf(a.ui[l] + pl, o);
+#pragma unroll
+    for (int l = 0; l < 3; ++l)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) g[l][m] = (double)ldf(a.g[l + 3 * m] + pl, o);
+    T nlt[3], p[6], sp[6];
+    dynm_adv(a, k, i, up, g, nlt);
+    dynm_products(a, k, up, p);
+    dynm_strain(a, k, g, sp, sf, sn);
+#pragma unroll
+    for (int l = 0; l < 3; ++l) stf(a.nlt[l] + pl, o, nlt[l]);
+    const double dl = a.delta[k];
+    const double nu = ct * dl * dl * (double)(T)sn;
+    const double su = 0.5 * a.ubarp[k];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+        const double tau = -2.0 * nu * ((double)sp[q] + (q == 2 ? su : 0.0));
+        stf(a.h[q] + pl, o, (T)(0.5 * (double)p[q] + tau));
+    }
+}
+
+// Stage 3 from u' and g' with the plane means.
+template <class T>
+__global__ void __launch_bounds__(256) k_dynm_plane3(DDims d, DynMixArgs<T> a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= d.nx) return;
+    const int nrows = d.ny * d.nzp;
+    for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
+        const int k = row / d.ny;
+        const unsigned o = ((unsigned)(row - k * d.ny) * (unsigned)d.nxpp + (unsigned)i) * (unsigned)sizeof(T);
+        dynm_tau_point(a, (size_t)k * d.ny * d.nxpp, o, k, i, a.cplane[k] / a.cplane[d.nzp + k]);
     }
 }
 
@@ -367,8 +514,8 @@ __global__ void __launch_bounds__(256) k_dynm_avg3(DDims d, DynMixArgs<T> A, con
             const int r = p / TX, c = p - r * TX;
             const int j = J0 + r, i = i0 + c;
             if (j < d.ny && i < d.nx) {
-                const unsigned o = (unsigned)(((k * d.ny + j) * d.nxpp + i) * (int)sizeof(T));
-                dynm_stage3_point(A, o, k, (double)(T)vn[m] / (double)(T)vd[m]);
+                const unsigned o = ((unsigned)j * (unsigned)d.nxpp + (unsigned)i) * (unsigned)sizeof(T);
+                dynm_tau_point(A, (size_t)k * plane, o, k, i, (double)(T)vn[m] / (double)(T)vd[m]);
             }
         }
     };
@@ -413,31 +560,83 @@ __global__ void __launch_bounds__(256) k_dynm_avg3(DDims d, DynMixArgs<T> A, con
     if (k1 == d.nzp) out(d.nzp - 1, Yc[0], Yc[1]);
 }
 
+// Planes per block of a pass that slides over z: each block takes two halo planes more, and a
+// last round of blocks costs as much as a full one (at_once blocks run at a time).  Measured
+// with 8 to 97 planes at 256x129x128 and 512x193x256: the choice was the fastest at both (the
+// slowest of them 10% and 3% of the step behind).
+static int slide_planes(long tiles, int nzp, long at_once) {
+    int best = nzp;
+    double cost = 1e300;
+    for (int nb = 1; nb <= (nzp + 3) / 4; ++nb) {
+        const int kc = (nzp + nb - 1) / nb;
+        const long blocks = tiles * ((nzp + kc - 1) / kc);
+        const double c = (double)((blocks + at_once - 1) / at_once) * (kc + 2);
+        if (c < cost) {
+            cost = c;
+            best = kc;
+        }
+    }
+    return best;
+}
+
 template <class T>
-int ph_dyn_mixed_avg3(lsb_ctx* c, const DynMixArgs<T>& a, hipStream_t s) {
-    const DDims d = ddims(c);
-    // 32-bit element offsets; the (1, 1) weights on the device
-    if ((double)d.ny * d.nzp * d.nxpp * sizeof(T) >= 2147483648.0 || a.cplane) return LSB_E_UNSUPPORTED;
-    const double* w = c->d_fz + 3 * c->nzp;  // the (1, 1) interpolating weights
-    constexpr int R = 4, TX = 128;
-    const int ntx = (d.nx + TX - 1) / TX;
+static void launch_dyn_test(lsb_ctx* c, const DDims& d, const DynMixArgs<T>& a, hipStream_t s) {
+    constexpr int R = 6;
+    const double* w = c->d_fz;  // the interpolating weights of the configured (a, b)
+    const double fa = c->cfg.a, fb = c->cfg.b;
+    int e = 0;
+    const bool p2 = std::frexp(2. * fa + fb, &e) == 0.5;
+    const int ntx = (d.nx + 61) / 62;
+    const int txo = (d.nx + ntx - 1) / ntx;
     const long tiles = (long)ntx * ((d.ny + R - 1) / R);
-    // 16 planes per block, fewer (each block recomputes two halo planes) until the grid
-    // holds some 2048 blocks (8 per CU)
-    int KC = 16;
-    while (KC > 4 && tiles * ((d.nzp + KC - 1) / KC) < 2048) KC /= 2;
-    const dim3 grid((unsigned)tiles, (unsigned)((d.nzp + KC - 1) / KC));
+    const int KC = slide_planes(tiles, d.nzp, 256);
+    const dim3 g((unsigned)tiles, (unsigned)((d.nzp + KC - 1) / KC));
+    if (p2)
+        hipLaunchKernelGGL((k_dynm_test<T, R, true>), g, dim3(64 * (R + 2)), 0, s, d, a, w, fa, fb, txo, KC);
+    else
+        hipLaunchKernelGGL((k_dynm_test<T, R, false>), g, dim3(64 * (R + 2)), 0, s, d, a, w, fa, fb, txo, KC);
+}
+
+template <class T>
+int ph_dyn_test(lsb_ctx* c, const DynMixArgs<T>& a, hipStream_t s) {
+    const DDims d = ddims(c);
     int tok = -1;
-    // num, den read; snorm, sp (6), h (6) read; h (6) written
-    prof_mark_begin(c, PC_NL, s, &tok, 0.0, 21.0 * sizeof(T) * (double)d.nx * d.ny * d.nzp);
-    hipLaunchKernelGGL((k_dynm_avg3<T, R, TX>), grid, dim3(256), 0, s, d, a, w, KC);
+    prof_mark_begin(c, PC_NL, s, &tok, 0.0, 14.0 * sizeof(T) * (double)d.nx * d.ny * d.nzp);
+    launch_dyn_test(c, d, a, s);
     prof_mark_end(c, tok, s);
     LSB_HIP(hipGetLastError());
     return LSB_OK;
 }
+template int ph_dyn_test<float>(lsb_ctx*, const DynMixArgs<float>&, hipStream_t);
+template int ph_dyn_test<double>(lsb_ctx*, const DynMixArgs<double>&, hipStream_t);
 
-template int ph_dyn_mixed_avg3<float>(lsb_ctx*, const DynMixArgs<float>&, hipStream_t);
-template int ph_dyn_mixed_avg3<double>(lsb_ctx*, const DynMixArgs<double>&, hipStream_t);
+// Stage 3 from num and den (their local average, or the plane means in a.cplane) and u', g'.
+template <class T>
+int ph_dyn_tau(lsb_ctx* c, const DynMixArgs<T>& a, hipStream_t s) {
+    const DDims d = ddims(c);
+    int tok = -1;
+    // num, den, u' and g' read; the N pieces and h written
+    prof_mark_begin(c, PC_NL, s, &tok, 0.0, 23.0 * sizeof(T) * (double)d.nx * d.ny * d.nzp);
+    if (a.cplane) {
+        hipLaunchKernelGGL((k_dynm_plane3<T>), row_grid(d), dim3(256), 0, s, d, a);
+    } else {
+        const double* w = c->d_fz + 3 * c->nzp;  // the (1, 1) interpolating weights
+        constexpr int R = 4, TX = 128;
+        const int ntx = (d.nx + TX - 1) / TX;
+        const long tiles = (long)ntx * ((d.ny + R - 1) / R);
+        // 16 planes per block, fewer (each block recomputes two halo planes) until the grid
+        // holds some 2048 blocks (8 per CU)
+        int KC = 16;
+        while (KC > 4 && tiles * ((d.nzp + KC - 1) / KC) < 2048) KC /= 2;
+        const dim3 grid((unsigned)tiles, (unsigned)((d.nzp + KC - 1) / KC));
+        hipLaunchKernelGGL((k_dynm_avg3<T, R, TX>), grid, dim3(256), 0, s, d, a, w, KC);
+    }
+    prof_mark_end(c, tok, s);
+    LSB_HIP(hipGetLastError());
+    return LSB_OK;
+}
+template int ph_dyn_tau<float>(lsb_ctx*, const DynMixArgs<float>&, hipStream_t);
+template int ph_dyn_tau<double>(lsb_ctx*, const DynMixArgs<double>&, hipStream_t);
 
 // Plane means of two fields over the nx physical points of every row: B partial sums per
 // plane (one block each), then the B partials of each plane summed in a fixed order.
@@ -501,12 +700,6 @@ template int ph_plane_mean2<float>(lsb_ctx*, const float*, const float*, double*
 
 size_t ph_plane_mean2_scratch(const lsb_ctx* c) { return (size_t)c->nzp * kPlaneBlocks * 2; }
 
-// LSB_NO_DYNX2=1: stages 1 and 2 one point per thread (for tests)
-static bool stage1_single() {
-    const char* e = std::getenv("LSB_NO_DYNX2");
-    return e && e[0] == '1';
-}
-
 template <class T>
 int ph_dyn_mixed(lsb_ctx* c, int stage, const DynMixArgs<T>& a, hipStream_t s) {
     const DDims d = ddims(c);
@@ -515,21 +708,8 @@ int ph_dyn_mixed(lsb_ctx* c, int stage, const DynMixArgs<T>& a, hipStream_t s) {
     // fields read + written per point by each stage
     const double per = (stage == 1) ? 12.0 + 22.0 : (stage == 2 ? 21.0 + 2.0 : 2.0 + 1.0 + 6.0 + 12.0);
     prof_mark_begin(c, PC_NL, s, &tok, 0.0, per * sizeof(T) * (double)d.nx * d.ny * d.nzp);
-    // 32-bit byte offsets while a field is below 4 GiB; FP32 two points per thread (8-byte
-    // accesses; FP64 has them with one)
+    // 32-bit byte offsets while a field is below 4 GiB
     const bool small = (double)d.ny * d.nzp * d.nxpp * sizeof(T) < 4294967296.0;
-    if constexpr (sizeof(T) == 4) {
-        if (stage != 3 && small && (d.nx % 2) == 0 && (d.nxpp % 2) == 0 && !stage1_single()) {
-            const dim3 g2((unsigned)((d.nx / 2 + 255) / 256), g.y);
-            if (stage == 1)
-                hipLaunchKernelGGL(k_dynm_stage1x2, g2, dim3(256), 0, s, d, a);
-            else
-                hipLaunchKernelGGL(k_dynm_stage2x2, g2, dim3(256), 0, s, d, a);
-            prof_mark_end(c, tok, s);
-            LSB_HIP(hipGetLastError());
-            return LSB_OK;
-        }
-    }
 #define LSB_DYNM(K)                                                          \
     if (small)                                                               \
         hipLaunchKernelGGL((K<T, unsigned>), g, dim3(256), 0, s, d, a);      \

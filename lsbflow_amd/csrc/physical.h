@@ -86,10 +86,12 @@ struct DynMixArgs {
 int ph_zero_pads(lsb_ctx* c, double* const* f, int nf, hipStream_t s);
 template <class T>
 int ph_dyn_mixed(lsb_ctx* c, int stage, const DynMixArgs<T>& a, hipStream_t s);
-// the (1, 1) average of num and den and stage 3 in one pass (numf, denf not written);
-// LSB_E_UNSUPPORTED where that pass does not apply (the caller runs the two steps)
+// the same in two passes that read u' and g': num and den with the test filter inside, then
+// stage 3 (and the N pieces) with the average of num and den inside
 template <class T>
-int ph_dyn_mixed_avg3(lsb_ctx* c, const DynMixArgs<T>& a, hipStream_t s);
+int ph_dyn_test(lsb_ctx* c, const DynMixArgs<T>& a, hipStream_t s);
+template <class T>
+int ph_dyn_tau(lsb_ctx* c, const DynMixArgs<T>& a, hipStream_t s);
 // out[k] = mean of f0 over plane k, out[nzp + k] = mean of f1 (nx physical points per row);
 // scratch: ph_plane_mean2_scratch(c) doubles
 template <class T>

@@ -468,11 +468,12 @@ int isc_full(lsb_ctx* c, double* ui, double* tau, double* work, hipStream_t s) {
     return sgs_interscale(c, u3, full_view(t9), work, s);
 }
 
-// Dynamic model of the step (sgsterm.f90:123-280), fields of T: products, strain and L1
-// (stage 1), the (a, b) test filter of S', L1, u', p, M:L and M:M (stage 2), their local
-// (1, 1) average or plane means, and h = p/2 + tau over the products (stage 3).  The work
-// fields follow each other in the SGS block.  An FP64 step at 512x193x256 takes 11.86 ms so,
-// and 12.24 with the products, strain, two averages and tau as passes of their own.
+// Dynamic model of the step (sgsterm.f90:123-280), fields of T: M:L and M:M from u' and g'
+// (the products, the strain, L1 and the (a, b) test filter inside), then their local (1, 1)
+// average or plane means, the N pieces and h = p/2 + tau.  LSB_NO_DYNFUSE=1 or
+// LSB_NO_DYNX2=1 (for tests): the stages and the filter as passes of their own, whose work
+// fields follow each other in the SGS block; the FP32 filter refuses nx > 1024 there, and
+// so does the mixed form's model.
 template <class T>
 static int dyn_step(lsb_ctx* c, StepState* S, hipStream_t s) {
     StepLayout& L = S->L;
@@ -510,6 +511,22 @@ static int dyn_step(lsb_ctx* c, StepState* S, hipStream_t s) {
     a.numf = W(36);
     a.denf = W(37);
     a.base = S->dynbase;
+    auto on = [](const char* name) {
+        const char* e = std::getenv(name);
+        return e && e[0] == '1';
+    };
+    // the plane means of num and den, for the plane-averaged coefficient
+    auto plane_mean = [&]() {
+        double* scr = reinterpret_cast<double*>(W(kDynWork));
+        double* cp = scr + ph_plane_mean2_scratch(c);
+        a.cplane = cp;
+        return ph_plane_mean2<T>(c, a.num, a.den, scr, cp, s);
+    };
+    if ((sizeof(T) == 8 || c->nx <= 1024) && !on("LSB_NO_DYNFUSE") && !on("LSB_NO_DYNX2")) {
+        LSB_TRY(ph_dyn_test(c, a, s));
+        if (c->cfg.dyn_avg) LSB_TRY(plane_mean());
+        return ph_dyn_tau(c, a, s);
+    }
     LSB_TRY(ph_dyn_mixed(c, 1, a, s));
     {
         const T* fi[21];
@@ -530,16 +547,8 @@ static int dyn_step(lsb_ctx* c, StepState* S, hipStream_t s) {
     }
     LSB_TRY(ph_dyn_mixed(c, 2, a, s));
     if (c->cfg.dyn_avg) {
-        double* scr = reinterpret_cast<double*>(W(kDynWork));
-        double* cp = scr + ph_plane_mean2_scratch(c);
-        LSB_TRY(ph_plane_mean2<T>(c, a.num, a.den, scr, cp, s));
-        a.cplane = cp;
+        LSB_TRY(plane_mean());
     } else {
-        // the (1, 1) average and stage 3 in one pass; LSB_NO_DYNFUSE=1 (for tests) or
-        // fields above 2 GiB: the averages through HBM, then stage 3
-        const char* e = std::getenv("LSB_NO_DYNFUSE");
-        const int rf = (e && e[0] == '1') ? LSB_E_UNSUPPORTED : ph_dyn_mixed_avg3(c, a, s);
-        if (rf != LSB_E_UNSUPPORTED) return rf;
         const T* fi[2] = {a.num, a.den};
         T* fo[2] = {W(36), W(37)};
         LSB_TRY(filter(fi, fo, 2, 1.0, 1.0));
