@@ -833,7 +833,7 @@ int fft_tune_y(lsb_ctx* c, void* work, hipStream_t s) {
         a.dt = c->dt;
         a.dtnui = 1.0;
         pick(TUNE_YRHS_F32, "yfwd+rhs f32", c32, 3, [&](int cc) {
-            return fast_yfwd_rhs(pc, np, lh, ny, (const cpx<float>*)hp.tw_y32, (float)scale, a, s, cc);
+            return fast_yfwd_rhs<float>(pc, np, lh, ny, (const cpx<float>*)hp.tw_y32, (float)scale, a, s, cc);
         });
     }
     (void)hipEventDestroy(e0);
@@ -871,25 +871,28 @@ template int horfft_xfwd<float>(lsb_ctx*, const HorPlan&, const float* const*, f
 
 // y pass of the three pieces of each N_l fused with the velocity right-hand side
 // (fast_yfwd_rhs); pieces[3 l + q] hold x-transformed rows.
-int horfft_yfwd_rhs(lsb_ctx* c, const HorPlan& hp, float* const* pieces, int nplanes, const YRhsArgs& a,
-                    hipStream_t s) {
+template <class T>
+int horfft_yfwd_rhs(lsb_ctx* c, const HorPlan& hp, T* const* pieces, int nplanes, const YRhsArgs& a, hipStream_t s) {
     if (!horfft_has_ops(hp)) {
         set_error("horfft (fused y pass): register-resident lengths nx/2 and ny");
         return LSB_E_UNSUPPORTED;
     }
-    FieldList<float> pc{};
+    FieldList<T> pc{};
     for (int q = 0; q < 9; ++q) pc.p[q] = pieces[q];
     int tok = -1;
     {
         const double pairs = (double)nplanes * hp.ny * hp.lh * 3.0;
-        const double per = 3.0 * 2 * sizeof(float) + 3.0 * 2 * sizeof(float) + 4.0 * 16.0;
+        const double per = 3.0 * 2 * sizeof(T) + 3.0 * 2 * sizeof(T) + 4.0 * 16.0;
         prof_mark_begin(c, PC_RHS, s, &tok, 9.0 * nplanes * 2.5 * hp.lh * hp.ny * std::log2((double)hp.ny),
                         pairs * per);
     }
-    LSB_TRY(fast_yfwd_rhs(pc, nplanes, hp.lh, hp.ny, (const cpx<float>*)hp.tw_y32,
-                          (float)(1.0 / ((double)hp.nx * hp.ny)), a, s, c->tune[TUNE_YRHS_F32]));
+    const cpx<T>* tw = (const cpx<T>*)(sizeof(T) == 8 ? (void*)hp.tw_y : (void*)hp.tw_y32);
+    LSB_TRY(fast_yfwd_rhs<T>(pc, nplanes, hp.lh, hp.ny, tw, (T)(1.0 / ((double)hp.nx * hp.ny)), a, s,
+                             sizeof(T) == 4 ? c->tune[TUNE_YRHS_F32] : 0));
     prof_mark_end(c, tok, s);
     return LSB_OK;
 }
+template int horfft_yfwd_rhs<double>(lsb_ctx*, const HorPlan&, double* const*, int, const YRhsArgs&, hipStream_t);
+template int horfft_yfwd_rhs<float>(lsb_ctx*, const HorPlan&, float* const*, int, const YRhsArgs&, hipStream_t);
 
 }  // namespace lsb

@@ -13,6 +13,7 @@ namespace lsb {
     LSB_MIXED_YFWD(extern, double, A, B)    \
     LSB_MIXED_YFWD(extern, float, A, B)     \
     LSB_MIXED_YINV(extern, double, A, B)    \
+    LSB_MIXED_YRHS(extern, double, A, B)    \
     LSB_MIXED_YRHS(extern, float, A, B)
 LSB_MIXED_CASES(X)
 #undef X
@@ -152,11 +153,11 @@ int fast_yinv3(const FieldList<double>& in, const FieldList<R>& out, int nplanes
     }
 }
 
-int fast_yfwd_rhs(const FieldList<float>& pieces, int nplanes, int lh, int ny, const cpx<float>* tw, float scale,
+template <class R>
+int fast_yfwd_rhs(const FieldList<R>& pieces, int nplanes, int lh, int ny, const cpx<R>* tw, R scale,
                   const YRhsArgs& a, hipStream_t s, int cols) {
     if (nplanes <= 0) return LSB_OK;
-    using R = float;
-    const int nc = ycols<R>(cols, ytile_cols<R>());
+    const int nc = ycols<R>(cols, 16);
     switch (ny) {
 #define CALL(A, B, C) launch_yrhs<R, R, A, B, C>(pieces, nplanes, lh, tw, scale, a, s)
 #define X(LL, A, B) LSB_YCASE(LL, (CALL(A, B, 8)), (CALL(A, B, 16)), (CALL(A, B, 32)))
@@ -179,7 +180,9 @@ int fast_yfwd_rhs(const FieldList<float>& pieces, int nplanes, int lh, int ny, c
     template int fast_yfwd<R>(const FieldList<R>&, const FieldList<R>&, int, int, int, int, const cpx<R>*, R,    \
                               hipStream_t, int);                                                                 \
     template int fast_yinv3<R>(const FieldList<double>&, const FieldList<R>&, int, int, int, int, int,           \
-                               const cpx<R>*, const double*, const double*, const double*, hipStream_t, int);
+                               const cpx<R>*, const double*, const double*, const double*, hipStream_t, int);   \
+    template int fast_yfwd_rhs<R>(const FieldList<R>&, int, int, int, const cpx<R>*, R, const YRhsArgs&,         \
+                                  hipStream_t, int);
 LSB_INST_FAST(double)
 LSB_INST_FAST(float)
 

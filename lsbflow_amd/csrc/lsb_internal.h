@@ -323,7 +323,8 @@ template <class T>
 int horfft_xfwd(lsb_ctx* c, const HorPlan& hp, const T* const* phys, T* const* rows, int nf, int nplanes,
                 hipStream_t s);
 struct YRhsArgs;
-int horfft_yfwd_rhs(lsb_ctx* c, const HorPlan& hp, float* const* pieces, int nplanes, const YRhsArgs& a,
+template <class T>
+int horfft_yfwd_rhs(lsb_ctx* c, const HorPlan& hp, T* const* pieces, int nplanes, const YRhsArgs& a,
                     hipStream_t s);
 // scratch: the y pass's staging buffer (nf * nplanes * ny * nx doubles) supplied by the
 // caller; null takes the context's staging slot 8 (allocated on first use); in_place: no
@@ -403,7 +404,8 @@ struct YRhsArgs {
     double* rhs[3];
     double ab0, ab1, ab2, bdf0, bdf1, bdf2, dt, dtnui;
 };
-int fast_yfwd_rhs(const FieldList<float>& pieces, int nplanes, int lh, int ny, const cpx<float>* tw, float scale,
+template <class R>
+int fast_yfwd_rhs(const FieldList<R>& pieces, int nplanes, int lh, int ny, const cpx<R>* tw, R scale,
                   const YRhsArgs& a, hipStream_t s, int cols = 0);
 // times the kx-column tiles of the y passes on this context's grid (scratch `work` of
 // at least 24 physical fields of doubles) and records the fastest in the tuning table

@@ -573,7 +573,7 @@ static int dyn_base_ready(lsb_ctx* c, StepState* S) {
 // N_l written to nlt (3 spectral).  Work comes from the step layout.
 // FP64 physical chain: inverse transforms, products + SGS model, forward transforms.
 static int nlterm_phys(lsb_ctx* c, StepState* S, const double* const* uif, double* nltf_out[3], double* hf[9],
-                       bool ops_on_load, const double* ftab, hipStream_t s) {
+                       bool ops_on_load, const double* ftab, bool xonly, hipStream_t s) {
     StepLayout& L = S->L;
     // inverse FFTs: ui (3) + g (9).  d/dz acts along pencils and commutes with the
     // horizontal transform, so with the register-resident FFT the z derivatives are
@@ -689,7 +689,11 @@ static int nlterm_phys(lsb_ctx* c, StepState* S, const double* const* uif, doubl
             in[n] = hph[q];
             out[n++] = hf[q];
         }
-        LSB_TRY(horfft_fwd(c, c->hp, in, out, n, c->nzp, s));
+        // xonly: the rows stay x-transformed for the fused y pass + right-hand side
+        if (xonly)
+            LSB_TRY(horfft_xfwd<double>(c, c->hp, in, out, n, c->nzp, s));
+        else
+            LSB_TRY(horfft_fwd(c, c->hp, in, out, n, c->nzp, s));
     }
     return LSB_OK;
 }
@@ -816,11 +820,7 @@ static int nlterm_core(lsb_ctx* c, StepState* S, const double* const* uif, doubl
         return LSB_E_ARG;
     }
     if (mixed_chain(c)) return nlterm_phys_mixed(c, S, uif, nltf_out, hf, ftab, xonly, s);
-    if (xonly) {
-        set_error("nlterm: the fused forward pass is built for the mixed form");
-        return LSB_E_ARG;
-    }
-    return nlterm_phys(c, S, uif, nltf_out, hf, ops_on_load, ftab, s);
+    return nlterm_phys(c, S, uif, nltf_out, hf, ops_on_load, ftab, xonly, s);
 }
 
 static void hf_view(StepState* S, bool sym, double* hf[9]) {
@@ -949,9 +949,11 @@ static int update_once(lsb_ctx* c) {
     double* hf[9];
     hf_view(S, sym, hf);
     double* nltf[3] = {L.spec[S_NLTF0], L.spec[S_NLTF0 + 1], L.spec[S_NLTF0 + 2]};
-    // mixed form on the register-resident FFT: the forward y pass of the N pieces is
-    // fused with the right-hand side (the transformed pieces stay in registers)
-    const bool fuse = mixed_form(c) && horfft_has_ops(c->hp) && sym;
+    // on the register-resident FFT the forward y pass of the N pieces is fused with the
+    // right-hand side (the transformed pieces stay in registers); LSB_NO_YRHS=1, for
+    // tests: the two passes
+    const char* no_yrhs = std::getenv("LSB_NO_YRHS");
+    const bool fuse = horfft_has_ops(c->hp) && sym && !(no_yrhs && no_yrhs[0] == '1');
     LSB_TRY(nlterm_core(c, S, uif, nltf, hf, ftab, s, fuse));
     // temperature part of the nonlinear term (navierstokes.f90:800-845)
     if (temp_on(c)) LSB_TRY(temp_nlterm(c, uif, ftab != nullptr, s));
@@ -997,7 +999,7 @@ static int update_once(lsb_ctx* c) {
         y.wavx = c->d_wavx;
         y.wavy = c->d_wavy;
         y.ubarpp = r.ubarpp;
-        float* pieces[9];
+        double* pieces[9];
         for (int l = 0; l < 3; ++l) {
             y.nout[l] = r.nout[l];
             y.nl[l] = r.nl[l];
@@ -1006,9 +1008,9 @@ static int update_once(lsb_ctx* c) {
             y.un[l] = r.un[l];
             y.unm[l] = r.unm[l];
             y.rhs[l] = r.rhs[l];
-            pieces[3 * l + 0] = reinterpret_cast<float*>(nltf[l]);
-            pieces[3 * l + 1] = reinterpret_cast<float*>(hf[l]);
-            pieces[3 * l + 2] = reinterpret_cast<float*>(hf[l + 3]);
+            pieces[3 * l + 0] = nltf[l];
+            pieces[3 * l + 1] = hf[l];
+            pieces[3 * l + 2] = hf[l + 3];
         }
         y.ab0 = r.ab0;
         y.ab1 = r.ab1;
@@ -1018,7 +1020,13 @@ static int update_once(lsb_ctx* c) {
         y.bdf2 = r.bdf2;
         y.dt = r.dt;
         y.dtnui = r.dtnui;
-        LSB_TRY(horfft_yfwd_rhs(c, c->hp, pieces, c->nzp, y, s));
+        if (mixed_form(c)) {
+            float* p32[9];
+            for (int q = 0; q < 9; ++q) p32[q] = reinterpret_cast<float*>(pieces[q]);
+            LSB_TRY(horfft_yfwd_rhs<float>(c, c->hp, p32, c->nzp, y, s));
+        } else {
+            LSB_TRY(horfft_yfwd_rhs<double>(c, c->hp, pieces, c->nzp, y, s));
+        }
     } else {
         LSB_TRY(sp_rhs_vel(c, r, s));
     }

@@ -133,3 +133,28 @@ def test_inverse_under_capture_without_staging():
         hip.lib.hipGraphDestroy(graph)
         for p in (spec, out, want):
             assert hip.lib.hipFree(p) == 0
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(32, 16, 16), (128, 64, 32), (512, 256, 16), (48, 24, 16), (180, 150, 16), (480, 240, 16)])
+def test_fp64_forward_y_with_rhs(nx, ny, nz, monkeypatch):
+    """The forward y pass with the right-hand side in its epilogue against the two passes
+    (LSB_NO_YRHS=1): the smallest, middle and largest lengths of both kinds, with partial
+    tiles of 16 kx columns, over three steps (each order of the schemes).  They differ by
+    roundings of the three pieces of N (a few 1e-16 of the largest, which the sum can leave
+    1e3 below): 1e-12 for N and the velocities; the pressure, a divergence divided by
+    k^2 dt, 1e-9."""
+    case = L.cases.CASES["c1_dns"].with_(name="yrhs", nx=nx, ny=ny, nz=nz, dt=1e-4, pert_rms=1e-2)
+    u, v, w = L.cases.initial_condition(case)
+    out = {}
+    for sep in ("0", "1"):
+        monkeypatch.setenv("LSB_NO_YRHS", sep)
+        c = setup_case(case)
+        try:
+            c.state_set(u, v, w)
+            c.timestep(3)
+            out[sep] = c.state_get()
+        finally:
+            c.close()
+    for k in ("uf", "vf", "wf", "pf", "nlnif", "nlnmif"):
+        assert np.all(np.isfinite(out["0"][k])), k
+        assert rel_l2(out["0"][k], out["1"][k]) < (1e-9 if k == "pf" else 1e-12), k
