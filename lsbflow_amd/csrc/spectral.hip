@@ -109,19 +109,22 @@ __global__ void k_specfilter(SpDims d, const double* __restrict__ tab, FieldList
     reinterpret_cast<c2*>(out.p[f])[q] = make_double2(re, im);
 }
 
-// horfft.f90:153-224 norm on the kx = 0 column and the ky-Nyquist row.
-// One thread per (field, z, j) with j in 0..ny-1 for the Nyquist row and the
-// symmetric pairs handled by the thread owning the lower index.
+// horfft.f90:153-224 norm on the kx = 0 column and the ky-Nyquist row (which no pair of the
+// column touches), in one launch: one thread per (field, z, j) of the column, the symmetric
+// pairs handled by the thread owning the lower index, then one per (field, z, i) of the row.
 __global__ void k_norm(FieldList<double> f, int nf, int nzp, int ny, int nx, int kx0_zero) {
     const int nyh = ny / 2;
-    const long n = (long)nf * nzp * ny;
+    const int per = ny + (ny > 2 ? nx : 0);
+    const long n = (long)nf * nzp * per;
     for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-        const int j = (int)(t % ny);
-        const long kf = t / ny;
+        const int j = (int)(t % per);
+        const long kf = t / per;
         const int k = (int)(kf % nzp);
         const int fi = (int)(kf / nzp);
         double* pl = f.p[fi] + (long)k * nx * ny;
-        if (kx0_zero) {
+        if (j >= ny) {
+            pl[(long)nyh * nx + (j - ny)] = 0.0;
+        } else if (kx0_zero) {
             if (j == 0) pl[1] = 0.0;
             if (ny > 2 && j >= 1 && j <= nyh - 1) {
                 const int jp = ny - j;  // 0-based partner of j (ny + 2 - (j+1) - 1)
@@ -135,17 +138,6 @@ __global__ void k_norm(FieldList<double> f, int nf, int nzp, int ny, int nx, int
                 b[1] = -im;
             }
         }
-    }
-}
-__global__ void k_norm_nyq(FieldList<double> f, int nf, int nzp, int ny, int nx) {
-    const int nyh = ny / 2;
-    const long n = (long)nf * nzp * nx;
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-        const int i = (int)(t % nx);
-        const long kf = t / nx;
-        const int k = (int)(kf % nzp);
-        const int fi = (int)(kf / nzp);
-        f.p[fi][((long)k * ny + nyh) * nx + i] = 0.0;
     }
 }
 
@@ -218,15 +210,10 @@ int sp_specfilter(lsb_ctx* c, const double* const* in, double* const* out, int n
 int sp_norm(lsb_ctx* c, double* const* f, int nf, hipStream_t s) {
     FieldList<double> fl{};
     for (int i = 0; i < nf; ++i) fl.p[i] = f[i];
-    const long n1 = (long)nf * c->nzp * c->ny;
+    const long n = (long)nf * c->nzp * (c->ny + (c->ny > 2 ? c->nx : 0));
     const int kx0 = (c->wavx[0] == 0.0) ? 1 : 0;
-    hipLaunchKernelGGL(k_norm, sp_grid(n1), dim3(256), 0, s, fl, nf, c->nzp, c->ny, c->nx, kx0);
+    hipLaunchKernelGGL(k_norm, sp_grid(n), dim3(256), 0, s, fl, nf, c->nzp, c->ny, c->nx, kx0);
     LSB_HIP(hipGetLastError());
-    if (c->ny > 2) {
-        const long n2 = (long)nf * c->nzp * c->nx;
-        hipLaunchKernelGGL(k_norm_nyq, sp_grid(n2), dim3(256), 0, s, fl, nf, c->nzp, c->ny, c->nx);
-        LSB_HIP(hipGetLastError());
-    }
     return LSB_OK;
 }
 
@@ -292,10 +279,49 @@ __global__ void k_rhs_vel(SpDims d, const double* __restrict__ wavx, const doubl
     }
 }
 
-// Boundary planes of the viscous step (navierstokes.f90:1321-1373), one thread
-// per (kx,ky) mode.  Writes bc_top[l], bc_bot[l] (one plane each).
-__global__ void k_bc_vel(SpDims d, const double* __restrict__ wavx, const double* __restrict__ wavy, StepBcArgs a) {
-    SP_LOOP(d.plane_pairs) {
+// Boundary planes of the viscous step (navierstokes.f90:1321-1373): bc_top[l], bc_bot[l]
+// (one plane each) and the scaled bound planes.  A block takes kBcPairs (kx, ky) modes:
+// kBcGroups groups of threads sum rows 0 and nzp-1 of d2w/dz2 over their share of the
+// planes, the groups' sums are added in a fixed order, then one thread per mode forms the
+// planes.  One launch for three (the two-row contraction, which the matrix kernel ran on
+// tiles of 64 rows, the bound scaling and this): bound by reading w once, 16 groups so that
+// small planes fill the chip too.  68 + 5 + 7 us before at 512x193x256, 28 + 5 + 6 at
+// 240x114x120; four 64x65x32 DNS steps 452 -> 390 us with it and the one-launch norm.
+constexpr int kBcPairs = 16;
+constexpr int kBcGroups = 16;
+__global__ void __launch_bounds__(kBcPairs * kBcGroups)
+    k_bc_vel(SpDims d, const double* __restrict__ wavx, const double* __restrict__ wavy, StepBcArgs a) {
+    __shared__ c2 part[2][kBcGroups][kBcPairs];
+    const int t = threadIdx.x % kBcPairs, grp = threadIdx.x / kBcPairs;
+    const long pr = (long)blockIdx.x * kBcPairs + t;
+    {
+        const c2* w = reinterpret_cast<const c2*>(a.w);
+        c2 st = make_double2(0.0, 0.0), sb = make_double2(0.0, 0.0);
+        if (pr < d.plane_pairs) {
+#pragma unroll 4
+            for (int k = grp; k < a.nzp; k += kBcGroups) {
+                const c2 v = w[(long)k * d.plane_pairs + pr];
+                const double mt = a.md2b[(long)k * kLdmBnd], mb = a.md2b[(long)k * kLdmBnd + 1];
+                st.x += mt * v.x;
+                st.y += mt * v.y;
+                sb.x += mb * v.x;
+                sb.y += mb * v.y;
+            }
+        }
+        part[0][grp][t] = st;
+        part[1][grp][t] = sb;
+    }
+    __syncthreads();
+    if (grp < 2) {
+        c2 v = part[grp][0][t];
+        for (int g = 1; g < kBcGroups; ++g) {
+            v.x += part[grp][g][t].x;
+            v.y += part[grp][g][t].y;
+        }
+        part[grp][0][t] = v;
+    }
+    __syncthreads();
+    if (grp == 0 && pr < d.plane_pairs) {
         const int m = (int)(pr % d.lh);
         const int j = (int)(pr / d.lh);
         const double wx = wavx[2 * m], wy = wavy[j];
@@ -334,12 +360,15 @@ __global__ void k_bc_vel(SpDims d, const double* __restrict__ wavx, const double
         reinterpret_cast<c2*>(a.bcb[0])[pr] = make_double2(dtb * (-wx * psi), dtb * (wx * psr));
         reinterpret_cast<c2*>(a.bcb[1])[pr] = make_double2(dtb * (-wy * psi), dtb * (wy * psr));
         // w: imposed field (bound) plus the Zang-Hussaini correction xnu*dt*bdfv*d2w/dz2
-        const c2 d2t = reinterpret_cast<const c2*>(a.d2w)[pr];                // row 0
-        const c2 d2b = reinterpret_cast<const c2*>(a.d2w)[d.plane_pairs + pr];  // row nzp-1
+        const c2 d2t = part[0][0][t];  // row 0
+        const c2 d2b = part[1][0][t];  // row nzp-1
         const double zh = a.xnu * a.dt * a.bdfv;
         if (a.nhom) {
-            const c2 gt = a.bnd_top ? reinterpret_cast<const c2*>(a.bnd_top)[pr] : make_double2(0.0, 0.0);
-            const c2 gb = a.bnd_bot ? reinterpret_cast<const c2*>(a.bnd_bot)[pr] : make_double2(0.0, 0.0);
+            const c2 ut = reinterpret_cast<const c2*>(a.bnd_top)[pr], ub = reinterpret_cast<const c2*>(a.bnd_bot)[pr];
+            const c2 gt = make_double2(a.ramp_top * ut.x, a.ramp_top * ut.y);
+            const c2 gb = make_double2(a.ramp_bot * ub.x, a.ramp_bot * ub.y);
+            reinterpret_cast<c2*>(a.sc_top)[pr] = gt;
+            reinterpret_cast<c2*>(a.sc_bot)[pr] = gb;
             reinterpret_cast<c2*>(a.bct[2])[pr] = make_double2(gt.x + zh * d2t.x, gt.y + zh * d2t.y);
             reinterpret_cast<c2*>(a.bcb[2])[pr] = gb;
         } else {
@@ -402,7 +431,8 @@ int sp_rhs_vel(lsb_ctx* c, const StepRhsArgs& a, hipStream_t s) {
 }
 int sp_bc_vel(lsb_ctx* c, const StepBcArgs& a, hipStream_t s) {
     SpDims d = sp_dims(c, 1);
-    hipLaunchKernelGGL(k_bc_vel, sp_grid(d.plane_pairs), dim3(256), 0, s, d, c->d_wavx, c->d_wavy, a);
+    hipLaunchKernelGGL(k_bc_vel, dim3((unsigned)((d.plane_pairs + kBcPairs - 1) / kBcPairs)),
+                       dim3(kBcPairs * kBcGroups), 0, s, d, c->d_wavx, c->d_wavy, a);
     LSB_HIP(hipGetLastError());
     return LSB_OK;
 }

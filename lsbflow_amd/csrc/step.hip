@@ -75,8 +75,8 @@ struct StepState {
     StepLayout L;
     // rotating spectral slots
     int u[3], un[3], unm[3], nl[3], nlm[3], nnew[3], rhs[4], p, pn;
-    // bc planes: bct[3], bcb[3], d2w (2), bnd_top, bnd_bot
-    double *bct[3], *bcb[3], *d2w, *bnd_top, *bnd_bot;
+    // bc planes: bct[3], bcb[3], bnd_top, bnd_bot
+    double *bct[3], *bcb[3], *bnd_top, *bnd_bot;
     double bnd00_top = 0.0, bnd00_bot = 0.0;  // (0,0) Re of the unit-amplitude bound planes
     // top_bc 2: the two difference planes, two physical scratch planes and the weight m(x)
     double *cdiff[2], *cphys[2], *cweight;
@@ -120,7 +120,7 @@ int step_alloc(lsb_ctx* c) {
     StepState* S = new StepState();
     const size_t ns = c->nspec, np = c->nphys, pl = c->plane_s;
     const int nsgs = sgs_fields(c);
-    const size_t nplanes = 6 + 2 + 2 + 2;
+    const size_t nplanes = 6 + 2 + 2;
     const size_t bytes =
         (NSPEC_SLOTS * ns + (NPHYS_SLOTS + nsgs) * np + nplanes * pl + 2 * c->plane_p + c->nx + 3 * c->nzp) *
         sizeof(double);
@@ -144,12 +144,11 @@ int step_alloc(lsb_ctx* c) {
         S->bct[l] = p + (size_t)l * pl;
         S->bcb[l] = p + (size_t)(3 + l) * pl;
     }
-    S->d2w = p + 6 * pl;
-    S->bnd_top = p + 8 * pl;
-    S->bnd_bot = p + 9 * pl;
-    S->cdiff[0] = p + 10 * pl;
-    S->cdiff[1] = p + 11 * pl;
-    S->cphys[0] = p + 12 * pl;
+    S->bnd_top = p + 6 * pl;
+    S->bnd_bot = p + 7 * pl;
+    S->cdiff[0] = p + 8 * pl;
+    S->cdiff[1] = p + 9 * pl;
+    S->cphys[0] = p + 10 * pl;
     S->cphys[1] = S->cphys[0] + c->plane_p;
     S->cweight = S->cphys[1] + c->plane_p;
     S->dynbase = S->cweight + c->nx;
@@ -306,14 +305,6 @@ int step_prepare(lsb_ctx* c) {
     StepState* S = state_of(c);
     if (!S) return LSB_E_STATE;
     return prepare_bound(c, S);
-}
-
-__global__ void k_scale2(const double* __restrict__ a, const double* __restrict__ b, double sa, double sb,
-                         double* __restrict__ oa, double* __restrict__ ob, long n) {
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-        oa[t] = sa * a[t];
-        ob[t] = sb * b[t];
-    }
 }
 
 // ------------------------------------------------------------ SGS drivers
@@ -1037,19 +1028,12 @@ static int update_once(lsb_ctx* c) {
     // with the sponge on (navierstokes.f90:1389)
     const bool nhom = (g.bctype > 0 && c->t >= g.istartbound);
     const bool vel_nhom = nhom || g.forcing == 1;
-    {
-        const double* in[1] = {L.spec[S->u[2]]};
-        double* out[1] = {S->d2w};
-        LSB_TRY(zcontract(c, c->d_md2b, kLdmBnd, 2, c->nzp, in, out, 1, s));
-    }
     const double ramp = bound_ramp(c, c->t);
     double st = ramp, sb = 0.0;
     if (g.bctype == 1) {
         const double bfac = (S->bnd00_bot != 0.0) ? (ramp * S->bnd00_top) / (ramp * S->bnd00_bot) : 0.0;
         sb = (ramp * S->bnd00_bot != 0.0) ? bfac * ramp : 0.0;
     }
-    double* bnd_t = S->L.planes + 6 * c->plane_s + 0;  // reuse d2w? no: separate scaled planes below
-    (void)bnd_t;
     double pfac0, pfac1;
     if (istep == 1) {
         pfac0 = 0.0;
@@ -1061,16 +1045,10 @@ static int update_once(lsb_ctx* c) {
         pfac0 = 2.0;
         pfac1 = -1.0;
     }
-    // scaled bound planes into bcb[2] / bct[2] happen inside the bc kernel via bnd_* pointers;
-    // the scale is applied to the stored unit planes first (into the hz scratch plane area)
-    double* sc_top = L.spec[S_DWDZ];                 // plane 0 of a free spectral slot
-    double* sc_bot = L.spec[S_DWDZ] + c->plane_s;    // plane 1
-    if (nhom) {
-        const long n = (long)c->plane_s;
-        hipLaunchKernelGGL(k_scale2, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, S->bnd_top, S->bnd_bot, st, sb,
-                           sc_top, sc_bot, n);
-        LSB_HIP(hipGetLastError());
-    }
+    // the bound planes times their factors (for w and the pressure step), two planes of a
+    // free spectral slot
+    double* sc_top = L.spec[S_DWDZ];
+    double* sc_bot = L.spec[S_DWDZ] + c->plane_s;
     StepBcArgs b{};
     b.rhs0 = L.spec[S->rhs[0]];
     b.rhs1 = L.spec[S->rhs[1]];
@@ -1081,9 +1059,15 @@ static int update_once(lsb_ctx* c) {
     b.top_bc = g.top_bc;
     b.cdiff[0] = S->cdiff[0];
     b.cdiff[1] = S->cdiff[1];
-    b.d2w = S->d2w;
-    b.bnd_top = nhom ? sc_top : nullptr;
-    b.bnd_bot = nhom ? sc_bot : nullptr;
+    b.w = L.spec[S->u[2]];
+    b.md2b = c->d_md2b;
+    b.nzp = c->nzp;
+    b.bnd_top = S->bnd_top;
+    b.bnd_bot = S->bnd_bot;
+    b.ramp_top = st;
+    b.ramp_bot = sb;
+    b.sc_top = sc_top;
+    b.sc_bot = sc_bot;
     for (int l = 0; l < 3; ++l) {
         b.bct[l] = S->bct[l];
         b.bcb[l] = S->bcb[l];
