@@ -19,7 +19,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "liblsbflow_amd.so")
 SOURCES = ["setup.cpp", "capi.cpp", "fft.hip", "fft_fast.hip", "fft_mixed_x64.hip", "fft_mixed_y64.hip",
-           "fft_mixed_x32.hip", "fft_mixed_y32.hip", "fft_mixed_r32.hip", "fft_mixed_r64.hip", "zops.hip", "spectral.hip", "physical.hip",
+           "fft_mixed_x32.hip", "fft_mixed_y32.hip", "fft_mixed_r32.hip", "fft_mixed_r64.hip", "fft_mixed_b64.hip", "zops.hip", "spectral.hip", "physical.hip",
            "step.hip", "dealias.hip", "iodiag.hip", "temperature.hip", "noalloc.hip", "dynamic.hip", "helmrefine.hip",
            "ensemble.hip"]
 ARCH = "gfx950"

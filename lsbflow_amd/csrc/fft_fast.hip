@@ -22,6 +22,10 @@ LSB_MIXED_CASES(X)
     LSB_MIXED_X(extern, float, A, B)
 LSB_MIXED_ODD_CASES(X)
 #undef X
+#define X(LL, A, B) LSB_MIXED_XBLEND(extern, A, B)
+LSB_MIXED_CASES(X)
+LSB_MIXED_ODD_CASES(X)
+#undef X
 
 bool pow2_fft_len(int L) { return L == 16 || L == 32 || L == 64 || L == 128 || L == 256; }
 
@@ -59,6 +63,20 @@ int fast_xinv(const FieldList<R>& in, const FieldList<R>& out, int nrows, int nf
     switch (lh) {
 #define X(LL, A, B) \
     case LL: return launch_xinv<R, R, R, A, B>(in, out, nrows, nf, istride, nxpp, tw, twr, s);
+        LSB_FAST_CASES(X)
+        LSB_MIXED_CASES(X)
+        LSB_MIXED_ODD_CASES(X)
+#undef X
+        default: return LSB_E_ARG;
+    }
+}
+
+int fast_xblend(const double* const* in, double* const* out, int ny, int lh, const double* m, const cpx<double>* tw,
+                const cpx<double>* twr, hipStream_t s) {
+    const XBlendArgs a{{in[0], in[1]}, {out[0], out[1]}, m, 1.0 / (2.0 * lh), ny};
+    switch (lh) {
+#define X(LL, A, B) \
+    case LL: return launch_xblend<double, A, B>(a, tw, twr, s);
         LSB_FAST_CASES(X)
         LSB_MIXED_CASES(X)
         LSB_MIXED_ODD_CASES(X)

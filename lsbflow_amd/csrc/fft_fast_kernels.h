@@ -25,6 +25,7 @@
 
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "lsb_internal.h"
 
@@ -794,7 +795,154 @@ __global__ void __launch_bounds__(C * N2) k_yfwd_rhs(FieldList<R> pc, int nplane
 }
 
 
+// The blended ceiling on one spectral plane, out += F[m(x) F^-1 in], in one launch: m
+// depends on x only, so the y transforms cancel.  Along x the rows ky and -ky of a real
+// field's half spectrum, F(kx, -ky) = conj F(-kx, ky), are two real lines,
+// P = (F(ky) + F(-ky)) / 2 and Q = (F(ky) - F(-ky)) / 2i: c2r, the weight (with the
+// transform pair's 1/nx in it) and r2c as in the x passes above, then P + iQ and P - iQ
+// are added to the two rows (ky = 0 and the Nyquist row pair with themselves, Q = 0).
+// Latency-bound: a plane or two, where the six launches of the 2-D transforms, the weight
+// and the sum took 30 us of a step.
+struct XBlendArgs {
+    const double* in[2];
+    double* out[2];
+    const double* m;
+    double scale;
+    int ny;
+};
+template <class R, int N1, int N2>
+__global__ void __launch_bounds__(kXLines<N2> * N2) k_xblend(XBlendArgs a, const cpx<R>* __restrict__ tw,
+                                                            const cpx<R>* __restrict__ twr) {
+    constexpr int L = N1 * N2;
+    constexpr int LPB = kXLines<N2>;
+    constexpr int NQ = kNQ<N1, N2>;
+    constexpr int TS = N1 * (N2 + 1);
+    static_assert(LPB % 2 == 0, "the two lines of a pair share a block");
+    __shared__ cpx<R> T[LPB * TS];
+    const int tid = threadIdx.x;
+    const int l = tid / N2, n2 = tid % N2;
+    const int nlines = a.ny + 2;
+    const int line = blockIdx.x * LPB + l;
+    const bool valid = line < nlines;
+    const int pr = min(line, nlines - 1) / 2;  // ky = pr and its partner
+    const bool isq = line & 1;
+    const int j0 = pr, j1 = (pr == 0) ? 0 : a.ny - pr;
+    const double* f = a.in[blockIdx.y];
+    const double* r0 = f + (long)j0 * (2 * L);
+    const double* r1 = f + (long)j1 * (2 * L);
+    cpx<R>* Tl = T + l * TS;
+    {
+        cpx<R> x[N1], y[N1];
+#pragma unroll
+        for (int j = 0; j < N1; ++j) {
+            x[j] = ld_c<R>(r0, n2 + N2 * j);
+            y[j] = ld_c<R>(r1, n2 + N2 * j);
+        }
+#pragma unroll
+        for (int j = 0; j < N1; ++j) {
+            const cpx<R> s = cadd(x[j], y[j]), d = csub(x[j], y[j]);
+            Tl[n2 + N2 * j] = isq ? cpx<R>{(R)0.5 * d.im, (R)-0.5 * d.re} : cpx<R>{(R)0.5 * s.re, (R)0.5 * s.im};
+        }
+    }
+    __syncthreads();
+    cpx<R> v[N1];
+#pragma unroll
+    for (int n1 = 0; n1 < N1; ++n1) {
+        const int n = N2 * n1 + n2;
+        cpx<R> xk = Tl[n];
+        cpx<R> xc;
+        if (n == 0) {
+            xk.im = 0;
+            xc = {0, 0};
+        } else {
+            xc = cconj(Tl[L - n]);
+        }
+        const cpx<R> s = cadd(xk, xc);
+        const cpx<R> d = csub(xk, xc);
+        const cpx<R> wd = cmul(cconj(twr[n]), d);
+        v[n1] = {s.re - wd.im, s.im + wd.re};
+    }
+    // the two stages of a transform of v through the line's tile, its outputs in u
+    cpx<R> u[NQ][N2];
+    auto stages = [&](auto sign) {
+        constexpr int S = decltype(sign)::value;
+        f_dft<R, S, N1>(v);
+        f_twiddle<R, S, N1>(v, n2, tw);
+        __syncthreads();
+#pragma unroll
+        for (int k1 = 0; k1 < N1; ++k1) Tl[k1 * (N2 + 1) + n2] = v[k1];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int k1 = n2 + N2 * q;
+            if (f_has_col<N1, N2>(k1)) {
+#pragma unroll
+                for (int j = 0; j < N2; ++j) u[q][j] = Tl[k1 * (N2 + 1) + j];
+                f_dft<R, S, N2>(u[q]);
+            }
+        }
+        __syncthreads();
+    };
+    stages(std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int k1 = n2 + N2 * q;
+        if (!f_has_col<N1, N2>(k1)) continue;
+#pragma unroll
+        for (int k2 = 0; k2 < N2; ++k2) {
+            const int k = k1 + N1 * k2;
+            Tl[k] = {u[q][k2].re * (R)(a.scale * a.m[2 * k]), u[q][k2].im * (R)(a.scale * a.m[2 * k + 1])};
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n1 = 0; n1 < N1; ++n1) v[n1] = Tl[N2 * n1 + n2];
+    stages(std::integral_constant<int, -1>{});
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+        if (f_has_col<N1, N2>(n2 + N2 * q)) {
+#pragma unroll
+            for (int k2 = 0; k2 < N2; ++k2) Tl[(n2 + N2 * q) + N1 * k2] = u[q][k2];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < N1; ++j) {
+        const int k = n2 + N2 * j;
+        const cpx<R> zk = Tl[k];
+        const cpx<R> zc = cconj(Tl[k == 0 ? 0 : L - k]);
+        const cpx<R> s = {(R)0.5 * (zk.re + zc.re), (R)0.5 * (zk.im + zc.im)};
+        const cpx<R> d = {(R)0.5 * (zk.re - zc.re), (R)0.5 * (zk.im - zc.im)};
+        const cpx<R> wd = cmul(twr[k], d);
+        v[j] = {s.re + wd.im, s.im - wd.re};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < N1; ++j) Tl[n2 + N2 * j] = v[j];
+    __syncthreads();
+    if (!valid || (isq && j0 == j1)) return;
+    const cpx<R>* Tp = T + (l ^ 1) * TS;  // the pair's other line
+    double* row = a.out[blockIdx.y] + (long)(isq ? j1 : j0) * (2 * L);
+#pragma unroll
+    for (int j = 0; j < N1; ++j) {
+        const int k = n2 + N2 * j;
+        const cpx<R> p = isq ? Tp[k] : v[j], q = isq ? v[j] : Tp[k];
+        const cpx<R> o = ld_c<R>(row, k);
+        // P + iQ or P - iQ
+        const cpx<R> x = isq ? cpx<R>{p.re + q.im, p.im - q.re} : cpx<R>{p.re - q.im, p.im + q.re};
+        st_c<R>(row, k, cadd(o, x));
+    }
+}
+
 // -------------------------------------------------------------- launchers
+template <class R, int N1, int N2>
+int launch_xblend(const XBlendArgs& a, const cpx<R>* tw, const cpx<R>* twr, hipStream_t s) {
+    constexpr int LPB = kXLines<N2>;
+    hipLaunchKernelGGL((k_xblend<R, N1, N2>), dim3((unsigned)((a.ny + 2 + LPB - 1) / LPB), 2), dim3(LPB * N2), 0, s, a,
+                       tw, twr);
+    LSB_HIP(hipGetLastError());
+    return LSB_OK;
+}
+
 template <class R, class TI, class TO, int N1, int N2>
 int launch_xfwd(const FieldList<TI>& in, const FieldList<TO>& out, int nrows, int nf, int istride, int ostride,
                 const cpx<R>* tw, const cpx<R>* twr, hipStream_t s) {
@@ -894,6 +1042,8 @@ constexpr int kMixedCols = 16;
                                                 const cpx<R>*, const cpx<R>*, hipStream_t);                      \
     E template int launch_xinv<R, R, R, N1, N2>(const FieldList<R>&, const FieldList<R>&, int, int, int, int,    \
                                                 const cpx<R>*, const cpx<R>*, hipStream_t);
+#define LSB_MIXED_XBLEND(E, N1, N2) \
+    E template int launch_xblend<double, N1, N2>(const XBlendArgs&, const cpx<double>*, const cpx<double>*, hipStream_t);
 #define LSB_MIXED_YINV3(E, R, N1, N2)                                                                            \
     E template int launch_yinv3<R, double, R, N1, N2, kMixedCols>(const FieldList<double>&, const FieldList<R>&, \
                                                                   int, int, int, int, const cpx<R>*,             \

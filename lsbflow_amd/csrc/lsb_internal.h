@@ -404,6 +404,9 @@ struct YRhsArgs {
     double* rhs[3];
     double ab0, ab1, ab2, bdf0, bdf1, bdf2, dt, dtnui;
 };
+// out[f] += F[m(x) F^-1 in[f]] on one spectral plane, f = 0, 1
+int fast_xblend(const double* const* in, double* const* out, int ny, int lh, const double* m, const cpx<double>* tw,
+                const cpx<double>* twr, hipStream_t s);
 template <class R>
 int fast_yfwd_rhs(const FieldList<R>& pieces, int nplanes, int lh, int ny, const cpx<R>* tw, R scale,
                   const YRhsArgs& a, hipStream_t s, int cols = 0);

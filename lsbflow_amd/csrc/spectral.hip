@@ -5,6 +5,7 @@
 // index like the reference (wavx(2m-1) = wavx(2m)), so kx(m) = wavx[2m].
 
 #include <cmath>
+#include <cstdlib>
 
 #include "lsb_internal.h"
 #include "spectral.h"
@@ -457,6 +458,11 @@ __global__ void k_add_planes(double* __restrict__ y0, double* __restrict__ y1, c
 int sp_ceiling_blend(lsb_ctx* c, double* const* bct, double* const* cdiff, double* const* phys, const double* m,
                      hipStream_t s) {
     const double* in[2] = {cdiff[0], cdiff[1]};
+    // LSB_NO_XBLEND=1 (for tests): the 2-D transforms
+    const char* e = std::getenv("LSB_NO_XBLEND");
+    if (horfft_has_ops(c->hp) && !(e && e[0] == '1'))
+        return fast_xblend(in, bct, c->ny, c->hp.lh, m, (const cpx<double>*)c->hp.tw_x,
+                           (const cpx<double>*)c->hp.tw_r, s);
     LSB_TRY(horfft_inv(c, c->hp, in, phys, 2, 1, s));
     const long np = (long)c->plane_p;
     hipLaunchKernelGGL(k_row_weight, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s, phys[0], phys[1], m, c->nx,
