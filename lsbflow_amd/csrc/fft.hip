@@ -409,6 +409,9 @@ static int lines_for(int len, size_t elem) {
     return l;
 }
 
+// whether the plan takes the register-resident passes for length len
+static bool plan_fast(const HorPlan& hp, int len) { return hp.pow2_only ? pow2_fft_len(len) : fast_fft_len(len); }
+
 static double fft_flops(const HorPlan& hp, int nf, int nplanes) {
     const double N = (double)hp.nx * hp.ny;
     return (double)nf * nplanes * 2.5 * N * std::log2(N);
@@ -434,7 +437,7 @@ int horfft_fwd(lsb_ctx* c, const HorPlan& hp, const double* const* phys, double*
     int tok = -1;
     prof_mark_begin(c, PC_FFT, s, &tok, fft_flops(hp, nf, nplanes), fft_bytes(hp, nf, nplanes, 8, 8));
     const int nrows = nplanes * ny;
-    if (fast_fft_len(lh)) {
+    if (plan_fast(hp, lh)) {
         LSB_TRY(fast_xfwd(in, out, nrows, nf, lh, nxpp, nx, (const cpx<double>*)hp.tw_x, (const cpx<double>*)hp.tw_r, s));
     } else {
         int lines = lines_for(lh, sizeof(cpx<double>));
@@ -445,7 +448,7 @@ int horfft_fwd(lsb_ctx* c, const HorPlan& hp, const double* const* phys, double*
         LSB_HIP(hipGetLastError());
     }
     const double scale = 1.0 / (double)(nx * ny);
-    if (fast_fft_len(ny)) {
+    if (plan_fast(hp, ny)) {
         LSB_TRY(fast_yfwd(out, out, nplanes, nf, lh, ny, (const cpx<double>*)hp.tw_y, scale, s, c->tune[TUNE_YFWD_F64]));
     } else {
         int cols = lines_for(ny, sizeof(cpx<double>));
@@ -460,7 +463,7 @@ int horfft_fwd(lsb_ctx* c, const HorPlan& hp, const double* const* phys, double*
     return LSB_OK;
 }
 
-bool horfft_has_ops(const HorPlan& hp) { return fast_fft_len(hp.ny) && fast_fft_len(hp.lh); }
+bool horfft_has_ops(const HorPlan& hp) { return plan_fast(hp, hp.ny) && plan_fast(hp, hp.lh); }
 bool horfft_needs_stage(const HorPlan& hp) { return pow2_fft_len(hp.ny) && pow2_fft_len(hp.lh); }
 
 // Whether the plain inverse stages its y pass in a compact buffer.  Powers of two always
@@ -515,7 +518,7 @@ int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, dou
         prof_mark_end(c, tok, s);
         return LSB_OK;
     }
-    if (fast_fft_len(ny)) {
+    if (plan_fast(hp, ny)) {
         LSB_TRY(fast_yinv(in, out, nplanes, nf, lh, ny, nxpp / 2, (const cpx<double>*)hp.tw_y, fo, c->d_wavx,
                           c->d_wavy, s));
     } else {
@@ -527,7 +530,7 @@ int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, dou
                            hp.py, (const cpx<double>*)hp.tw_y, cols);
         LSB_HIP(hipGetLastError());
     }
-    if (fast_fft_len(lh)) {
+    if (plan_fast(hp, lh)) {
         LSB_TRY(fast_xinv(out, out, nrows, nf, lh, nxpp, nxpp, (const cpx<double>*)hp.tw_x,
                           (const cpx<double>*)hp.tw_r, s));
     } else {

@@ -77,6 +77,8 @@ struct HorPlan {
     float* tw_x32 = nullptr;
     float* tw_y32 = nullptr;
     float* tw_r32 = nullptr;
+    // the lengths with a factor 3 or 5 stay on the Stockham passes
+    bool pow2_only = false;
 };
 
 // A list of field base pointers passed by value to batched kernels.

@@ -281,46 +281,48 @@ __global__ void k_rhs_vel(SpDims d, const double* __restrict__ wavx, const doubl
 }
 
 // Boundary planes of the viscous step (navierstokes.f90:1321-1373): bc_top[l], bc_bot[l]
-// (one plane each) and the scaled bound planes.  A block takes kBcPairs (kx, ky) modes:
-// kBcGroups groups of threads sum rows 0 and nzp-1 of d2w/dz2 over their share of the
-// planes, the groups' sums are added in a fixed order, then one thread per mode forms the
+// (one plane each) and the scaled bound planes.  A block takes kBcPairs (kx, ky) modes: its
+// threads bring kBcPlanes planes of w at a time into LDS, 64 of them sum rows 0 and nzp-1 of
+// d2w/dz2 plane by plane (the matrix kernel's order), then one thread per mode forms the
 // planes.  One launch for three (the two-row contraction, which the matrix kernel ran on
-// tiles of 64 rows, the bound scaling and this): bound by reading w once, 16 groups so that
-// small planes fill the chip too.  68 + 5 + 7 us before at 512x193x256, 28 + 5 + 6 at
-// 240x114x120; four 64x65x32 DNS steps 452 -> 390 us with it and the one-launch norm.
+// tiles of 64 rows, the bound scaling and this): bound by reading w once, with 8 loads a
+// thread in flight on 16 modes a block so that small planes fill the chip too.  68 + 5 + 7 us
+// before at 512x193x256, 28 + 5 + 6 at 240x114x120; four 64x65x32 DNS steps 452 -> 390 us
+// with it and the one-launch norm.
 constexpr int kBcPairs = 16;
 constexpr int kBcGroups = 16;
+constexpr int kBcPlanes = 128;
 __global__ void __launch_bounds__(kBcPairs * kBcGroups)
     k_bc_vel(SpDims d, const double* __restrict__ wavx, const double* __restrict__ wavy, StepBcArgs a) {
-    __shared__ c2 part[2][kBcGroups][kBcPairs];
+    __shared__ c2 tile[kBcPlanes][kBcPairs];
+    __shared__ double rows[kBcPlanes][2];
+    __shared__ c2 part[2][kBcPairs];
     const int t = threadIdx.x % kBcPairs, grp = threadIdx.x / kBcPairs;
     const long pr = (long)blockIdx.x * kBcPairs + t;
-    {
-        const c2* w = reinterpret_cast<const c2*>(a.w);
-        c2 st = make_double2(0.0, 0.0), sb = make_double2(0.0, 0.0);
-        if (pr < d.plane_pairs) {
-#pragma unroll 4
-            for (int k = grp; k < a.nzp; k += kBcGroups) {
-                const c2 v = w[(long)k * d.plane_pairs + pr];
-                const double mt = a.md2b[(long)k * kLdmBnd], mb = a.md2b[(long)k * kLdmBnd + 1];
-                st.x += mt * v.x;
-                st.y += mt * v.y;
-                sb.x += mb * v.x;
-                sb.y += mb * v.y;
-            }
+    const long prc = pr < d.plane_pairs ? pr : d.plane_pairs - 1;  // modes past the end read the last one
+    const c2* w = reinterpret_cast<const c2*>(a.w);
+    const int comp = threadIdx.x & 1, row = (threadIdx.x >> 1) & 1, mode = threadIdx.x >> 2;
+    double sum = 0.0;
+    for (int k0 = 0; k0 < a.nzp; k0 += kBcPlanes) {
+        const int n = min(kBcPlanes, a.nzp - k0);
+        c2 v[kBcPlanes / kBcGroups];
+#pragma unroll
+        for (int q = 0; q < kBcPlanes / kBcGroups; ++q)
+            v[q] = w[(long)(k0 + min(grp + kBcGroups * q, n - 1)) * d.plane_pairs + prc];
+        if (threadIdx.x < 2 * kBcPlanes) {
+            const int k = threadIdx.x >> 1;
+            if (k < n) rows[k][threadIdx.x & 1] = a.md2b[(long)(k0 + k) * kLdmBnd + (threadIdx.x & 1)];
         }
-        part[0][grp][t] = st;
-        part[1][grp][t] = sb;
-    }
-    __syncthreads();
-    if (grp < 2) {
-        c2 v = part[grp][0][t];
-        for (int g = 1; g < kBcGroups; ++g) {
-            v.x += part[grp][g][t].x;
-            v.y += part[grp][g][t].y;
+#pragma unroll
+        for (int q = 0; q < kBcPlanes / kBcGroups; ++q) tile[grp + kBcGroups * q][t] = v[q];
+        __syncthreads();
+        if (threadIdx.x < 4 * kBcPairs) {
+#pragma unroll 8
+            for (int k = 0; k < n; ++k) sum = fma(rows[k][row], comp ? tile[k][mode].y : tile[k][mode].x, sum);
         }
-        part[grp][0][t] = v;
+        __syncthreads();
     }
+    if (threadIdx.x < 4 * kBcPairs) (comp ? part[row][mode].y : part[row][mode].x) = sum;
     __syncthreads();
     if (grp == 0 && pr < d.plane_pairs) {
         const int m = (int)(pr % d.lh);
@@ -361,8 +363,8 @@ __global__ void __launch_bounds__(kBcPairs * kBcGroups)
         reinterpret_cast<c2*>(a.bcb[0])[pr] = make_double2(dtb * (-wx * psi), dtb * (wx * psr));
         reinterpret_cast<c2*>(a.bcb[1])[pr] = make_double2(dtb * (-wy * psi), dtb * (wy * psr));
         // w: imposed field (bound) plus the Zang-Hussaini correction xnu*dt*bdfv*d2w/dz2
-        const c2 d2t = part[0][0][t];  // row 0
-        const c2 d2b = part[1][0][t];  // row nzp-1
+        const c2 d2t = part[0][t];  // row 0
+        const c2 d2b = part[1][t];  // row nzp-1
         const double zh = a.xnu * a.dt * a.bdfv;
         if (a.nhom) {
             const c2 ut = reinterpret_cast<const c2*>(a.bnd_top)[pr], ub = reinterpret_cast<const c2*>(a.bnd_bot)[pr];
