@@ -243,7 +243,7 @@ __device__ __forceinline__ double lane_next(double v) {
 // 14 field passes in place of 99; bound by the vector units (some 410 instructions per point
 // and plane, 4/3 of the x phase for the halo rows) with HBM close behind.  R = 6: 8 waves
 // with up to 256 registers (42 FP64 values of the z pass each); R = 4 and R = 10 leave 168 and spill (FP64
-// step at 512x193x256: 8.36 ms against 10.6 and 13.3).  At that grid 1.07 ms in place of
+// step at 512x193x256: 8.36 ms against 10.6 and 13.3).  At that grid 1.13 ms in place of
 // 1.62 + 2.08 + 0.94 for stage 1, the filter and stage 2.
 template <class T, int R, bool P2>
 __global__ void __launch_bounds__(64 * (R + 2)) k_dynm_test(DDims d, DynMixArgs<T> A, const double* __restrict__ w,
