@@ -185,6 +185,7 @@ int upload_context(lsb_ctx* c) {
             LSB_HIP(hipMemcpyAsync(c->d_walls, walls.data(), walls.size() * sizeof(int), hipMemcpyHostToDevice, s));
         LSB_HIP(hipStreamSynchronize(s));
     }
+    LSB_TRY(step_base_upload(c));
     LSB_HIP(hipStreamSynchronize(s));
     return LSB_OK;
 }

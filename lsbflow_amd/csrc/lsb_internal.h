@@ -464,6 +464,8 @@ int ph_sgs(lsb_ctx* c, int model, const double* ui, const double* uiuj, const do
 
 // step (step.hip)
 int step_alloc(lsb_ctx* c);
+// base-flow profiles of the step's dynamic model, where there is a state block
+int step_base_upload(lsb_ctx* c);
 int step_run(lsb_ctx* c, int nsteps, bool with_norm);
 // graph capture of the step (ensemble.hip): one step enqueued with its host bookkeeping,
 // the bookkeeping alone, the slot-rotation period, and whether a step can be captured

@@ -115,6 +115,15 @@ static int sgs_fields(const lsb_ctx* c) {
     }
 }
 
+// The dynamic model's z-filtered base profiles, uploaded when the state block is made and
+// whenever the base flow or the filter weights are (upload_context): every path that steps,
+// captured graphs too, finds those of the present base flow.
+static int base_upload(lsb_ctx* c, StepState* S) {
+    if (c->cfg.sgsflag != 1 || c->cfg.sgsmodel != 1) return LSB_OK;
+    dyn_base_profiles(c, S->dynbase_h);
+    return upload(S->dynbase, S->dynbase_h.data(), S->dynbase_h.size() * sizeof(double), c->stream);
+}
+
 int step_alloc(lsb_ctx* c) {
     if (state_of(c)) return LSB_OK;
     StepState* S = new StepState();
@@ -160,6 +169,7 @@ int step_alloc(lsb_ctx* c) {
             m[i] = std::exp(-(e * e));
         }
         int ru = upload(S->cweight, m.data(), m.size() * sizeof(double), c->stream);
+        if (ru == LSB_OK) ru = base_upload(c, S);
         if (ru != LSB_OK) {
             delete S;
             return ru;
@@ -179,6 +189,11 @@ int step_alloc(lsb_ctx* c) {
     S->pn = S_PN;
     g_states.push_back({c, S});
     return LSB_OK;
+}
+
+int step_base_upload(lsb_ctx* c) {
+    StepState* S = state_of(c);
+    return S ? base_upload(c, S) : LSB_OK;
 }
 
 double* step_field(lsb_ctx* c, int which) {
@@ -547,18 +562,6 @@ static int dyn_step(lsb_ctx* c, StepState* S, hipStream_t s) {
     return ph_dyn_mixed(c, 3, a, s);
 }
 
-// the dynamic model's z-filtered base profiles, uploaded where the base flow has changed
-static int dyn_base_ready(lsb_ctx* c, StepState* S) {
-    if (c->cfg.sgsflag != 1 || c->cfg.sgsmodel != 1) return LSB_OK;
-    std::vector<double> h;
-    dyn_base_profiles(c, h);
-    if (h == S->dynbase_h) return LSB_OK;
-    S->dynbase_h.swap(h);
-    LSB_HIP(hipMemcpyAsync(S->dynbase, S->dynbase_h.data(), S->dynbase_h.size() * sizeof(double),
-                           hipMemcpyHostToDevice, c->stream));
-    return LSB_OK;
-}
-
 // ------------------------------------------------------- nonlinear term
 // navierstokes.f90:658-795 for T = 0: uif (3 spectral, already filtered) ->
 // N_l written to nlt (3 spectral).  Work comes from the step layout.
@@ -829,7 +832,6 @@ int nlterm_dev(lsb_ctx* c, const double* const* uif, double* const* nlt, hipStre
     LSB_TRY(step_alloc(c));
     StepState* S = state_of(c);
     const bool sym = !(c->cfg.sgsflag == 1 && c->cfg.sgsmodel == 3);
-    LSB_TRY(dyn_base_ready(c, S));
     double* hf[9];
     hf_view(S, sym, hf);
     double* nltf[3] = {S->L.spec[S_NLTF0], S->L.spec[S_NLTF0 + 1], S->L.spec[S_NLTF0 + 2]};
@@ -1176,7 +1178,6 @@ int step_run(lsb_ctx* c, int nsteps, bool with_norm) {
         set_error("timestep: the context belongs to a captured ensemble; step it with lsb_ensemble_timestep");
         return LSB_E_STATE;
     }
-    LSB_TRY(dyn_base_ready(c, S));
     for (int n = 0; n < nsteps; ++n) {
         if (with_norm) {
             LSB_TRY(step_enqueue(c));

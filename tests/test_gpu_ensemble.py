@@ -125,3 +125,40 @@ def test_smallest_uneven_member_against_oracle():
     g["_sens"] = {k: rel_l2(st2[k], st[k]) for k in ("uf", "vf", "wf", "pf")}
     print(f"{small.name} {small.nx}x{small.nzp}x{small.ny}:", flush=True)
     check_fields(st, g)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_base_flow_of_captured_dynamic_member(precision):
+    """The dynamic model's filtered base profiles follow the base flow into captured steps: a
+    member whose base flow and state are set after its last eager step, then captured, and
+    whose base flow changes again between graph launches, against eager steps (bit-equal)."""
+    case = members_small()[2]
+    u, v, w = L.cases.initial_condition(case)
+    flows = [tuple(f * b for b in L.cases.base_flow(case)) for f in (1.0, 0.7, 1.2)]
+
+    def resume(c, g, flow):
+        c.set_paral(*flow)
+        c.state_set(*(g[k] for k in FIELDS), istep=g["istep"], t=g["t"])
+
+    ref, c = setup_case(case, precision=precision), setup_case(case, precision=precision)
+    try:
+        for x in (ref, c):
+            x.state_set(u, v, w)
+            x.timestep(3)
+        start = c.state_get()
+        for x in (ref, c):
+            resume(x, start, flows[1])
+        with Ensemble([c]) as ens:
+            for flow in (flows[1], flows[2]):
+                ref.set_paral(*flow)
+                c.set_paral(*flow)
+                ref.timestep(4)
+                ens.timestep(4)
+                ens.synchronize()
+                g, r = c.state_get(), ref.state_get()
+                for k in FIELDS:
+                    assert np.all(np.isfinite(r[k])), k
+                    assert np.array_equal(g[k], r[k]), k
+    finally:
+        c.close()
+        ref.close()
