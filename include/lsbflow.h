@@ -401,7 +401,10 @@ int lsb_set_adaptive_dt(lsb_ctx* ctx, int dtadapt, int iomod, double fsize);
 
 /* ------------------------------------- device-pointer kernel entry points */
 /* Same semantics as the tier-A routines, on device memory, asynchronous on
- * `stream` (NULL = the context stream). */
+ * `stream` (NULL = the context stream).  The inverse transform where nx/2 and ny are both
+ * powers of two (16 to 256) stages a pass in a buffer of the context, allocated on first
+ * use: such calls of one context must not overlap (two streams, two threads, or beside a
+ * step), nor a call need a larger buffer than a graph captured it with. */
 int lsb_horfft_dev(lsb_ctx* ctx, double* ain, double* ainf, int is, int nfields, void* stream);
 int lsb_dfdz_dev(lsb_ctx* ctx, const double* uf, double* dudzf, int nfields, void* stream);
 int lsb_solve_helmholtz_dev(lsb_ctx* ctx, double* rhs, double dtnui, int nfields, void* stream);
@@ -423,12 +426,13 @@ int lsb_solve_helmholtz_mixed_dev(lsb_ctx* ctx, double* rhs, double dtnui, int n
 /* lsb_horfft_dev without device allocation.  No counterpart in the reference: it is
  * for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  Same arguments and results as
- * lsb_horfft_dev; the inverse transform's staging buffer is a library-owned device
- * array of 256 MiB per GPU (2^25 doubles; resolved by lsb_create, held until the
- * process ends) instead of a buffer allocated on first use, and the call makes no
- * hipMalloc/hipFree.  LSB_E_ARG when one field's staging (nzp*ny*nx doubles) exceeds
- * the array; fields are transformed in batches that fit it.  All calls on one GPU
- * share the array: calls that overlap on a GPU (two streams, two threads) race. */
+ * lsb_horfft_dev; the staging buffer of the inverse transform with power-of-two nx/2 and
+ * ny is a library-owned device array of 256 MiB per GPU (2^25 doubles; resolved by
+ * lsb_create, held until the process ends) instead of a buffer allocated on first use,
+ * and the call makes no hipMalloc/hipFree.  There LSB_E_ARG when one field's staging
+ * (nzp*ny*nx doubles) exceeds the array; fields are transformed in batches that fit it.
+ * All such calls on one GPU share the array: calls that overlap on a GPU (two streams,
+ * two threads) race.  The other lengths take no buffer. */
 int lsb_horfft_dev_noalloc(lsb_ctx* ctx, double* ain, double* ainf, int is, int nfields, void* stream);
 
 /* Kernel timing for roofline accounting.  Between lsb_profile_begin and

@@ -15,6 +15,7 @@
 // Each workgroup keeps its lines in LDS and runs a mixed-radix Stockham
 // sequence; twiddles come from tables computed in long double on the host.
 
+#include <algorithm>
 #include <cmath>
 
 #include <cstdio>
@@ -466,23 +467,19 @@ int horfft_fwd(lsb_ctx* c, const HorPlan& hp, const double* const* phys, double*
 bool horfft_has_ops(const HorPlan& hp) { return plan_fast(hp, hp.ny) && plan_fast(hp, hp.lh); }
 bool horfft_needs_stage(const HorPlan& hp) { return pow2_fft_len(hp.ny) && pow2_fft_len(hp.lh); }
 
-// Whether the plain inverse stages its y pass in a compact buffer.  Powers of two always
-// have.  The lengths with a factor 3 or 5 transform in place in the padded rows, as the
-// LDS path does, while the fields stay in the 256 MB last-level cache (240 x 114 x 120, 3
-// fields: 59 us against 56 us staged; 480 x 193 x 240, 1 field: 128 against 142), and
-// stage above it (3 fields: 385 us against 550); also in place where the buffer would
-// have to be allocated under a stream capture or while an ensemble's graphs hold it.
-static bool inv_staged(const lsb_ctx* c, const HorPlan& hp, size_t bytes, hipStream_t s) {
-    if (horfft_needs_stage(hp)) return true;
-    if (bytes <= (size_t)256 << 20) return false;
-    if (c->stage_bytes.size() > 8 && c->stage_bytes[8] >= bytes) return true;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cs) != hipSuccess) return false;
-    return cs == hipStreamCaptureStatusNone && !c->stage_locked;
-}
+// The inverse at the lengths with a factor 3 or 5 takes no buffer that a caller's graph,
+// another stream or another thread could share: pieces of at most kInvPiece bytes go through
+// both passes in turn, each with its y pass staged, compact and on 128-byte lines, in output
+// that a later piece is going to write (a piece is no larger than the next), the last in
+// place in its padded rows.  Bound by the copy rate of the 256 MB last-level cache and of
+// HBM; us with pieces (with all fields in place at once; with a staging buffer of their
+// size): 3 fields of 480x193x240 432 (547; 385), 1 of 480x366x240 266 (345; 251), 16 of
+// 240x114x120 317 (435; 301), 12 of 180x301x60 246 (319; 271).  Pieces of 64 to 160 MB take
+// 4-24% longer, of 256 MB up to 12%.
+constexpr size_t kInvPiece = (size_t)192 << 20;
 
 int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, double* const* phys, int nf,
-                   int nplanes, const int* ops, hipStream_t s, double* scratch, bool in_place) {
+                   int nplanes, const int* ops, hipStream_t s, double* scratch) {
     if (nf < 1 || nf > kMaxFields) {
         set_error("horfft: 1..16 fields per launch");
         return LSB_E_ARG;
@@ -505,7 +502,7 @@ int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, dou
     prof_mark_begin(c, PC_FFT, s, &tok, fft_flops(hp, nf, nplanes), fft_bytes(hp, nf, nplanes, 8, 8));
     const int nrows = nplanes * ny;
     const size_t per = (size_t)nplanes * ny * nx;
-    if (horfft_has_ops(hp) && !in_place && (scratch || inv_staged(c, hp, per * nf * sizeof(double), s))) {
+    if (horfft_needs_stage(hp)) {
         // y pass into a compact scratch (rows of lh complex, 128-byte aligned), then the
         // x pass out of place into the padded physical rows
         void* scr = scratch;
@@ -515,6 +512,34 @@ int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, dou
         LSB_TRY(fast_yinv(in, mid, nplanes, nf, lh, ny, lh, (const cpx<double>*)hp.tw_y, fo, c->d_wavx, c->d_wavy, s));
         LSB_TRY(fast_xinv(mid, out, nrows, nf, lh, nx, nxpp, (const cpx<double>*)hp.tw_x, (const cpx<double>*)hp.tw_r,
                           s));
+        prof_mark_end(c, tok, s);
+        return LSB_OK;
+    }
+    if (horfft_has_ops(hp)) {
+        const size_t splane = (size_t)nx * ny, pplane = (size_t)nxpp * ny;
+        const int budget = (int)std::clamp<size_t>(kInvPiece / (pplane * sizeof(double)), 1, 1 << 20);  // planes
+        // pieces of whole fields, or of one field's planes; the first ones are the smaller
+        const int kp = (nplanes + budget - 1) / budget;
+        const int fp = kp > 1 ? nf : (nf + budget / nplanes - 1) / (budget / nplanes);
+        const auto start = [](int n, int p, int i) { return n / p * i + std::max(0, i - (p - n % p)); };
+        for (int i = 0; i < fp * kp; ++i) {
+            const int f0 = start(nf, fp, i / kp), pf = start(nf, fp, i / kp + 1) - f0;
+            const int k0 = start(nplanes, kp, i % kp), pk = start(nplanes, kp, i % kp + 1) - k0;
+            const bool last = i + 1 == fp * kp, next_field = k0 + pk == nplanes;
+            FieldList<double> pin{}, mid{}, pout{};
+            FftOps po{};
+            for (int f = 0; f < pf; ++f) {
+                pin.p[f] = in.p[f0 + f] + splane * k0;
+                pout.p[f] = out.p[f0 + f] + pplane * k0;
+                po.op[f] = fo.op[f0 + f];
+                double* room = last ? pout.p[f] : next_field ? out.p[f0 + pf + f] : pout.p[f] + pplane * pk;
+                mid.p[f] = last ? room : (double*)(((uintptr_t)room + 127) & ~(uintptr_t)127);
+            }
+            LSB_TRY(fast_yinv(pin, mid, pk, pf, lh, ny, last ? nxpp / 2 : lh, (const cpx<double>*)hp.tw_y, po,
+                              c->d_wavx, c->d_wavy, s));
+            LSB_TRY(fast_xinv(mid, pout, pk * ny, pf, lh, last ? nxpp : nx, nxpp, (const cpx<double>*)hp.tw_x,
+                              (const cpx<double>*)hp.tw_r, s));
+        }
         prof_mark_end(c, tok, s);
         return LSB_OK;
     }

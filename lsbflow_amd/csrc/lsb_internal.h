@@ -319,7 +319,7 @@ int horfft_inv(lsb_ctx* c, const HorPlan& hp, const double* const* spec, double*
                int nplanes, hipStream_t s);
 // inverse with per-field d/dx, d/dy applied on load (FOP_*); fast lengths only
 bool horfft_has_ops(const HorPlan& hp);
-// whether the inverse has always staged its y pass (powers of two)
+// whether the plain inverse stages its y pass in a compact buffer (powers of two)
 bool horfft_needs_stage(const HorPlan& hp);
 template <class T>
 int horfft_xfwd(lsb_ctx* c, const HorPlan& hp, const T* const* phys, T* const* rows, int nf, int nplanes,
@@ -329,10 +329,10 @@ template <class T>
 int horfft_yfwd_rhs(lsb_ctx* c, const HorPlan& hp, T* const* pieces, int nplanes, const YRhsArgs& a,
                     hipStream_t s);
 // scratch: the y pass's staging buffer (nf * nplanes * ny * nx doubles) supplied by the
-// caller; null takes the context's staging slot 8 (allocated on first use); in_place: no
-// staging, the y pass writes the padded rows
+// caller, used where horfft_needs_stage; null takes the context's staging slot 8 (allocated
+// on first use)
 int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, double* const* phys, int nf,
-                   int nplanes, const int* ops, hipStream_t s, double* scratch = nullptr, bool in_place = false);
+                   int nplanes, const int* ops, hipStream_t s, double* scratch = nullptr);
 // allocation-free entry points (noalloc.hip): resolve the device address of the
 // file-scope scratch array on `device` (the current device); called by lsb_create
 int noalloc_resolve(int device);

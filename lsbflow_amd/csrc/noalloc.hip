@@ -69,20 +69,18 @@ extern "C" int lsb_horfft_dev_noalloc(lsb_ctx* c, double* ain, double* ainf, int
         return LSB_E_STATE;
     }
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
-    // fields per launch: the inverse y pass stages nzp * ny * nx doubles per field
-    // (powers of two; the lengths with a factor 3 or 5 go without where it does not fit)
+    // fields per launch: the inverse y pass of the powers of two stages nzp * ny * nx doubles
+    // per field
     int batch = kMaxFields;
-    bool in_place = false;
-    if (is == 1 && horfft_has_ops(c->hp)) {
+    if (is == 1 && horfft_needs_stage(c->hp)) {
         const size_t per = (size_t)c->nzp * c->ny * c->nx;
-        in_place = per > kScratchDoubles && !horfft_needs_stage(c->hp);
-        if (per > kScratchDoubles && !in_place) {
+        if (per > kScratchDoubles) {
             set_error("horfft_dev_noalloc: one field (" + std::to_string(per * 8) +
                       " bytes of staging) exceeds the scratch maximum of " + std::to_string(kScratchDoubles * 8) +
                       " bytes");
             return LSB_E_ARG;
         }
-        if (!in_place) batch = (int)std::min<size_t>((size_t)kMaxFields, kScratchDoubles / per);
+        batch = (int)std::min<size_t>((size_t)kMaxFields, kScratchDoubles / per);
     }
     for (int f0 = 0; f0 < nfields; f0 += batch) {
         const int nb = std::min(batch, nfields - f0);
@@ -100,7 +98,7 @@ extern "C" int lsb_horfft_dev_noalloc(lsb_ctx* c, double* ain, double* ainf, int
         if (is == -1)
             LSB_TRY(horfft_fwd(c, c->hp, pin, pout, nb, c->nzp, s));
         else
-            LSB_TRY(horfft_inv_ops(c, c->hp, pin, pout, nb, c->nzp, nullptr, s, scr, in_place));
+            LSB_TRY(horfft_inv_ops(c, c->hp, pin, pout, nb, c->nzp, nullptr, s, scr));
     }
     return LSB_OK;
 }

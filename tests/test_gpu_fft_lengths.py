@@ -87,8 +87,8 @@ def test_mixed_step_against_fp64(nx, ny):
 
 
 def test_noalloc_beyond_its_scratch_stays_accepted():
-    """One field of 480 x 240 x 301 exceeds the 2^25-double scratch: the lengths with a
-    factor 3 or 5 transform in place there, to the staged route's bits."""
+    """One field of 480 x 240 x 301 exceeds the 2^25-double scratch, which the lengths with a
+    factor 3 or 5 do not use: accepted, the bits of lsb_horfft_dev."""
     nx, ny, nz = 480, 240, 300
     hip, lib = Hip(), _lib.lib()
     with Context(Config(nx=nx, ny=ny, nz=nz)) as ctx:
@@ -106,33 +106,104 @@ def test_noalloc_beyond_its_scratch_stays_accepted():
     assert np.array_equal(*got)
 
 
-def test_inverse_under_capture_without_staging():
-    """A first inverse transform inside a stream capture allocates nothing at these lengths,
-    also beyond the size from which it stages its y pass (one field of 337 MB): it runs in
-    place in the output rows, and the graph replays to the eager, staged bits."""
+def device_fields(hip, nf, nx, ny, nzp, seed):
+    """(nf spectral fields on the device, room for their physical ones, its shape)"""
+    s = np.random.default_rng(seed).standard_normal((nf, nzp, ny, nx))
+    shape = (nf, nzp, ny, nx + 2)
+    spec, out = hip.alloc(s.nbytes), hip.alloc(8 * int(np.prod(shape)))
+    hip.put(spec, s)
+    hip.put(out, np.zeros(shape))
+    return spec, out, shape
+
+
+def capture(hip, stream, enqueue):
+    graph, ex = C.c_void_p(), C.c_void_p()
+    assert hip.lib.hipStreamBeginCapture(stream, 1) == 0
+    enqueue()
+    assert hip.lib.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.lib.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+    assert hip.lib.hipGraphDestroy(graph) == 0
+    return ex
+
+
+@pytest.mark.parametrize("nz,nf", [(100, 3), (250, 2)])
+def test_inverse_takes_no_memory(nz, nf):
+    """Three fields of 93 MB (a piece of one field and one of two) and two of 232 MB (two pieces
+    of the planes of each) leave the device's free memory as it was, and have the bits of
+    fifty planes at a time."""
+    nx, ny, np50 = 480, 240, 50
+    hip, lib = Hip(), _lib.lib()
+    with Context(Config(nx=nx, ny=ny, nz=nz)) as ctx, Context(Config(nx=nx, ny=ny, nz=np50 - 1)) as few:
+        spec, out, shape = device_fields(hip, nf, nx, ny, nz + 1, 3)
+        for f in range(nf):
+            for k in range(0, nz, np50):
+                o, i = (C.c_void_p(p.value + 8 * (f * (nz + 1) + k) * ny * n) for p, n in ((out, nx + 2), (spec, nx)))
+                _lib.check(lib.lsb_horfft_dev(few.h, o, i, 1, 1, None), "horfft")
+        few.synchronize()
+        want = hip.get(out, shape)[:, :nz]
+        hip.put(out, np.zeros(shape))
+        free = hip.free_bytes()
+        _lib.check(lib.lsb_horfft_dev(ctx.h, out, spec, 1, nf, None), "horfft")
+        ctx.synchronize()
+        assert hip.free_bytes() == free
+        assert np.array_equal(hip.get(out, shape)[:, :nz], want)
+        for p in (spec, out):
+            assert hip.lib.hipFree(p) == 0
+
+
+def test_first_inverse_under_capture():
+    """A first inverse transform inside a stream capture, one field of 337 MB (two pieces of
+    its planes): the graph replays to the eager bits."""
     nx, ny, nz = 480, 240, 365
     hip, lib = Hip(), _lib.lib()
-    shape = (nz + 1, ny, nx + 2)
     with Context(Config(nx=nx, ny=ny, nz=nz)) as ctx, Context(Config(nx=nx, ny=ny, nz=nz)) as ref:
-        s = np.random.default_rng(5).standard_normal((nz + 1, ny, nx))
-        spec, out, want = hip.alloc(s.nbytes), hip.alloc(8 * np.prod(shape)), hip.alloc(8 * np.prod(shape))
-        hip.put(spec, s)
+        spec, out, shape = device_fields(hip, 1, nx, ny, nz + 1, 5)
+        want = hip.alloc(8 * int(np.prod(shape)))
         _lib.check(lib.lsb_horfft_dev(ref.h, want, spec, 1, 1, None), "horfft")
         ref.synchronize()
-        stream, graph, ex = C.c_void_p(ctx.stream()), C.c_void_p(), C.c_void_p()
-        assert hip.lib.hipStreamBeginCapture(stream, 1) == 0
-        _lib.check(lib.lsb_horfft_dev(ctx.h, out, spec, 1, 1, stream), "horfft")
-        assert hip.lib.hipStreamEndCapture(stream, C.byref(graph)) == 0
-        assert hip.lib.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+        stream = C.c_void_p(ctx.stream())
+        ex = capture(hip, stream, lambda: _lib.check(lib.lsb_horfft_dev(ctx.h, out, spec, 1, 1, stream), "horfft"))
         for _ in range(3):
             hip.put(out, np.zeros(shape))
             assert hip.lib.hipGraphLaunch(ex, stream) == 0
             ctx.synchronize()
             assert np.array_equal(hip.get(out, shape), hip.get(want, shape))
         hip.lib.hipGraphExecDestroy(ex)
-        hip.lib.hipGraphDestroy(graph)
         for p in (spec, out, want):
             assert hip.lib.hipFree(p) == 0
+
+
+def test_captured_inverse_outlives_larger_calls():
+    """A graph of the inverse captured after an eager one of the same size (280 MB) replays to
+    the eager bits also after eager calls with more fields, and beside a transform of the same
+    context on another stream: it holds no buffer of the context."""
+    nx, ny, nz = 480, 240, 100
+    hip, lib = Hip(), _lib.lib()
+
+    def inverse(ctx, f, nf, stream):
+        _lib.check(lib.lsb_horfft_dev(ctx.h, f[1], f[0], 1, nf, stream), "horfft")
+
+    with Context(Config(nx=nx, ny=ny, nz=nz)) as ctx, Context(Config(nx=nx, ny=ny, nz=nz)) as other:
+        a, b = (device_fields(hip, nf, nx, ny, nz + 1, 10 + nf) for nf in (3, 4))
+        s1, s2 = C.c_void_p(ctx.stream()), C.c_void_p(other.stream())
+        inverse(ctx, a, 3, s1)
+        inverse(ctx, b, 4, s1)
+        ctx.synchronize()
+        want = [hip.get(x[1], x[2]) for x in (a, b)]
+        ex = capture(hip, s1, lambda: inverse(ctx, a, 3, s1))
+        for _ in range(3):
+            for x in (a, b):
+                hip.put(x[1], np.zeros(x[2]))
+            assert hip.lib.hipGraphLaunch(ex, s1) == 0
+            inverse(ctx, b, 4, s2)
+            ctx.synchronize()
+            other.synchronize()
+            for x, w in zip((a, b), want):
+                assert np.array_equal(hip.get(x[1], x[2]), w)
+        hip.lib.hipGraphExecDestroy(ex)
+        for x in (a, b):
+            for p in x[:2]:
+                assert hip.lib.hipFree(p) == 0
 
 
 @pytest.mark.parametrize("nx,ny,nz", [(32, 16, 16), (128, 64, 32), (512, 256, 16), (48, 24, 16), (180, 150, 16), (480, 240, 16)])
