@@ -138,8 +138,9 @@ extern "C" int lsb_ensemble_create(lsb_ctx** members, int n, lsb_ensemble** out)
     e->join.assign(n, nullptr);
     for (int i = 0; i < n && rc == LSB_OK; ++i)
         if (hipEventCreateWithFlags(&e->join[i], hipEventDisableTiming) != hipSuccess) rc = LSB_E_HIP;
+    if (rc != LSB_OK) set_error("ensemble_create: stream / event creation failed");
+    for (int i = 0; i < n && rc == LSB_OK; ++i) rc = step_reserve(e->m[i]);
     if (rc != LSB_OK) {
-        set_error("ensemble_create: stream / event creation failed");
         release(e);
         delete e;
         return rc;

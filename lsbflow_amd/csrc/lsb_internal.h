@@ -468,9 +468,10 @@ int step_alloc(lsb_ctx* c);
 int step_base_upload(lsb_ctx* c);
 int step_run(lsb_ctx* c, int nsteps, bool with_norm);
 // graph capture of the step (ensemble.hip): one step enqueued with its host bookkeeping,
-// the bookkeeping alone, the slot-rotation period, and whether a step can be captured
+// the bookkeeping alone, the buffers to hold before, the slot-rotation period, and whether a step can be captured
 int step_enqueue(lsb_ctx* c);
 void step_host_advance(lsb_ctx* c);
+int step_reserve(lsb_ctx* c);
 int step_rotation_period(lsb_ctx* c);
 bool step_capturable(const lsb_ctx* c, std::string& why);
 int step_prepare(lsb_ctx* c);

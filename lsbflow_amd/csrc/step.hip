@@ -1168,6 +1168,15 @@ static void rotate_slots(StepState* S) {
     S->pn = op;
 }
 
+// The FP64 chain's staging at the lengths with a factor 3 or 5 (the fused gradient transform,
+// slot 8), for a step that is captured before an eager one has allocated it.  The powers of
+// two and the mixed chain refuse such a capture (the staging is locked by then).
+int step_reserve(lsb_ctx* c) {
+    if (mixed_chain(c) || !horfft_has_ops(c->hp) || horfft_needs_stage(c->hp)) return LSB_OK;
+    void* p = nullptr;
+    return stage_get(c, 8, c->nspec * 9 * sizeof(double), &p);
+}
+
 int step_run(lsb_ctx* c, int nsteps, bool with_norm) {
     StepState* S = state_of(c);
     if (!S || !c->state_ready) {

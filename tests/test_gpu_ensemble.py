@@ -162,3 +162,27 @@ def test_base_flow_of_captured_dynamic_member(precision):
     finally:
         c.close()
         ref.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(48, 24), (96, 30), (40, 18)])
+def test_ensemble_of_resumed_members(nx, ny):
+    """An FP64 member resumed past its start-up steps (lsb_state_set with istep 3) and captured
+    without an eager step of its own, at lengths with a factor 3 or 5: captured as it is, and
+    bit-equal to eager steps."""
+    case = members_small()[1].with_(name="resumed", nx=nx, ny=ny, dealiasflag=0)
+    first = eager(case, 0, 3)
+    c, ref = setup_case(case), setup_case(case)
+    try:
+        for x in (c, ref):
+            x.state_set(*(first[k] for k in FIELDS), istep=first["istep"], t=first["t"])
+        ref.timestep(5)
+        with Ensemble([c]) as ens:
+            ens.timestep(5)
+            ens.synchronize()
+            g, r = c.state_get(), ref.state_get()
+        for k in FIELDS:
+            assert np.all(np.isfinite(r[k])), k
+            assert np.array_equal(g[k], r[k]), k
+    finally:
+        c.close()
+        ref.close()
