@@ -80,8 +80,10 @@ struct StepState {
     double bnd00_top = 0.0, bnd00_bot = 0.0;  // (0,0) Re of the unit-amplitude bound planes
     // top_bc 2: the two difference planes, two physical scratch planes and the weight m(x)
     double *cdiff[2], *cphys[2], *cweight;
-    // dynamic model: z-filtered base profiles (3 nzp) and their host copy
+    // dynamic model: z-filtered base profiles (3 nzp) and their host copy; the plane means of
+    // M:L and M:M (2 nzp) and their partial sums
     double* dynbase = nullptr;
+    double* dynmean = nullptr;
     std::vector<double> dynbase_h;
 };
 
@@ -102,14 +104,10 @@ void step_free(lsb_ctx* c) {
         }
 }
 
-// dynamic model work fields (symmetric): snorm, 5 x 6 tensors, uihat (3), num/den and filtered
-// (4); then the two-pass filter's intermediate fields
-constexpr int kDynWork = 1 + 6 * 5 + 3 + 4;
-
 static int sgs_fields(const lsb_ctx* c) {
     if (!c->cfg.sgsflag) return 0;
     switch (c->cfg.sgsmodel) {
-        case 1: return kDynWork + kMaxFields;
+        case 1: return 2;                 // M:L and M:M
         case 3: return 24 + 9 + 9;        // ub, ub2, uibuj, filtered; filter tmp (9); tau (9)
         default: return 0;
     }
@@ -130,9 +128,9 @@ int step_alloc(lsb_ctx* c) {
     const size_t ns = c->nspec, np = c->nphys, pl = c->plane_s;
     const int nsgs = sgs_fields(c);
     const size_t nplanes = 6 + 2 + 2;
-    const size_t bytes =
-        (NSPEC_SLOTS * ns + (NPHYS_SLOTS + nsgs) * np + nplanes * pl + 2 * c->plane_p + c->nx + 3 * c->nzp) *
-        sizeof(double);
+    const size_t bytes = (NSPEC_SLOTS * ns + (NPHYS_SLOTS + nsgs) * np + nplanes * pl + 2 * c->plane_p + c->nx +
+                          (3 + 2) * c->nzp + ph_plane_mean2_scratch(c)) *
+                         sizeof(double);
     void* blk = nullptr;
     int rc = dev_alloc(&blk, bytes);
     if (rc != LSB_OK) {
@@ -161,6 +159,7 @@ int step_alloc(lsb_ctx* c) {
     S->cphys[1] = S->cphys[0] + c->plane_p;
     S->cweight = S->cphys[1] + c->plane_p;
     S->dynbase = S->cweight + c->nx;
+    S->dynmean = S->dynbase + 3 * c->nzp;
     {   // inflow weight of the ceiling: the blowing Gaussian of the bctype 3 profile
         std::vector<double> m(c->nx);
         const double L = c->cfg.xlen;
@@ -476,26 +475,21 @@ int isc_full(lsb_ctx* c, double* ui, double* tau, double* work, hipStream_t s) {
 
 // Dynamic model of the step (sgsterm.f90:123-280), fields of T: M:L and M:M from u' and g'
 // (the products, the strain, L1 and the (a, b) test filter inside), then their local (1, 1)
-// average or plane means, the N pieces and h = p/2 + tau.  LSB_NO_DYNFUSE=1 or
-// LSB_NO_DYNX2=1 (for tests): the stages and the filter as passes of their own, whose work
-// fields follow each other in the SGS block; the FP32 filter refuses nx > 1024 there, and
-// so does the mixed form's model.
+// average or plane means, the N pieces and h = p/2 + tau.  LSB_NO_DYNFUSE=1 (for tests): the
+// stages and the filter as passes of their own, their work fields in staging slot 23.  The
+// mixed form's model refuses nx > 1024, as its FP32 filter does.
 template <class T>
 static int dyn_step(lsb_ctx* c, StepState* S, hipStream_t s) {
+    if (sizeof(T) == 4 && c->nx > 1024) {
+        set_error("dynamic model (mixed form): needs nx <= 1024");
+        return LSB_E_UNSUPPORTED;
+    }
     StepLayout& L = S->L;
     auto ph = [&](int slot) { return reinterpret_cast<T*>(L.phys[slot]); };
-    auto W = [&](int i) { return reinterpret_cast<T*>(L.sgs) + (size_t)i * c->nphys; };
-    auto filter = [&](const T* const* in, T* const* out, int nf, double fa, double fb) {
-        if constexpr (sizeof(T) == 4)
-            return ph_filter3_f32(c, in, out, nf, fa, fb, s);
-        else
-            return ph_filter3(c, in, out, nf, fa, fb, 1, W(kDynWork), s);
-    };
     DynMixArgs<T> a{};
     for (int l = 0; l < 3; ++l) {
         a.ui[l] = ph(P_UI0 + l);
         a.nlt[l] = ph(P_NLT0 + l);
-        a.uh[l] = W(25 + l);
     }
     for (int q = 0; q < 9; ++q) a.g[q] = ph(P_G0 + q);
     a.ubar = c->d_paral;
@@ -505,34 +499,44 @@ static int dyn_step(lsb_ctx* c, StepState* S, hipStream_t s) {
     for (int q = 0; q < 6; ++q) {
         a.p[q] = ph(P_H0 + q);
         a.h[q] = ph(P_H0 + q);
+    }
+    a.num = reinterpret_cast<T*>(L.sgs);
+    a.den = a.num + c->nphys;
+    a.base = S->dynbase;
+    // the plane means of num and den, for the plane-averaged coefficient
+    auto plane_mean = [&]() {
+        a.cplane = S->dynmean;
+        return ph_plane_mean2<T>(c, a.num, a.den, S->dynmean + 2 * c->nzp, S->dynmean, s);
+    };
+    const char* sep = std::getenv("LSB_NO_DYNFUSE");
+    if (!(sep && sep[0] == '1')) {
+        LSB_TRY(ph_dyn_test(c, a, s));
+        if (c->cfg.dyn_avg) LSB_TRY(plane_mean());
+        return ph_dyn_tau(c, a, s);
+    }
+    // S' (6), L1 (6), |S|, their filtered values and those of u' and p (21), the averages (2);
+    // then the two-pass filter's intermediate fields
+    constexpr int kDynWork = 6 + 6 + 1 + 21 + 2;
+    void* work = nullptr;
+    LSB_TRY(stage_get(c, 23, (size_t)(kDynWork + kMaxFields) * c->nphys * sizeof(T), &work));
+    auto W = [&](int i) { return reinterpret_cast<T*>(work) + (size_t)i * c->nphys; };
+    auto filter = [&](const T* const* in, T* const* out, int nf, double fa, double fb) {
+        if constexpr (sizeof(T) == 4)
+            return ph_filter3_f32(c, in, out, nf, fa, fb, s);
+        else
+            return ph_filter3(c, in, out, nf, fa, fb, 1, W(kDynWork), s);
+    };
+    for (int q = 0; q < 6; ++q) {
         a.sp[q] = W(q);
         a.l1[q] = W(6 + q);
         a.sph[q] = W(13 + q);
         a.l1h[q] = W(19 + q);
         a.ph[q] = W(28 + q);
     }
+    for (int l = 0; l < 3; ++l) a.uh[l] = W(25 + l);
     a.snorm = W(12);
-    a.num = W(34);
-    a.den = W(35);
-    a.numf = W(36);
-    a.denf = W(37);
-    a.base = S->dynbase;
-    auto on = [](const char* name) {
-        const char* e = std::getenv(name);
-        return e && e[0] == '1';
-    };
-    // the plane means of num and den, for the plane-averaged coefficient
-    auto plane_mean = [&]() {
-        double* scr = reinterpret_cast<double*>(W(kDynWork));
-        double* cp = scr + ph_plane_mean2_scratch(c);
-        a.cplane = cp;
-        return ph_plane_mean2<T>(c, a.num, a.den, scr, cp, s);
-    };
-    if ((sizeof(T) == 8 || c->nx <= 1024) && !on("LSB_NO_DYNFUSE") && !on("LSB_NO_DYNX2")) {
-        LSB_TRY(ph_dyn_test(c, a, s));
-        if (c->cfg.dyn_avg) LSB_TRY(plane_mean());
-        return ph_dyn_tau(c, a, s);
-    }
+    a.numf = W(34);
+    a.denf = W(35);
     LSB_TRY(ph_dyn_mixed(c, 1, a, s));
     {
         const T* fi[21];
@@ -556,7 +560,7 @@ static int dyn_step(lsb_ctx* c, StepState* S, hipStream_t s) {
         LSB_TRY(plane_mean());
     } else {
         const T* fi[2] = {a.num, a.den};
-        T* fo[2] = {W(36), W(37)};
+        T* fo[2] = {W(34), W(35)};
         LSB_TRY(filter(fi, fo, 2, 1.0, 1.0));
     }
     return ph_dyn_mixed(c, 3, a, s);

@@ -7,6 +7,7 @@ import pytest
 import lsbflow_amd as L
 from lsbflow_amd._lib import LsbError
 from lsbflow_amd.core import setup_case
+from tests.test_zz_no_alloc import Hip
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +48,21 @@ def test_two_passes_bit_identical(nx, ny, nz, b, dyn_avg, forcing, precision, mo
     for k in ("uf", "vf", "wf", "pf", "nlnif", "nlnmif"):
         assert np.all(np.isfinite(out["0"][k])), k
         assert np.array_equal(out["0"][k], out["1"][k]), k
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_state_holds_what_the_two_passes_use(precision):
+    """The dynamic model's state takes three fields more than the sigma model's (M:L, M:M and
+    the plane means' partial sums); allocations are rounded, one field at most."""
+    hip, taken = Hip(), []
+    for model in (2, 1):
+        case = L.cases.CASES["c2_dyn_les"].with_(name="mem", nx=128, ny=64, nz=64, sgsmodel=model)
+        with setup_case(case, precision=precision) as c:
+            before = hip.free_bytes()
+            c.state_set(*L.cases.initial_condition(case))
+            c.timestep(2)
+            c.synchronize()
+            taken.append(before - hip.free_bytes())
+    field = 130 * 64 * 65 * 8
+    print(f"precision {precision}: {(taken[1] - taken[0]) / field:.1f} fields", flush=True)
+    assert taken[1] - taken[0] <= 4 * field

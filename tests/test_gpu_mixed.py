@@ -127,8 +127,8 @@ def test_mixed_dynamic_small(dyn_avg):
 @pytest.mark.parametrize("nx,ny,nz", [(128, 64, 64), (96, 30, 64), (512, 32, 64), (512, 256, 128)])
 def test_mixed_dynamic_fused_average_bit_identical(nx, ny, nz, monkeypatch):
     """The local (1, 1) average of M:L and M:M and stage 3 in one pass give the same bits as
-    the averages through HBM followed by stage 3 (LSB_NO_DYNFUSE=1): a register-resident
-    grid, a generic one whose tiles are partial in x and y (nx = 96, ny = 30), a grid of
+    the averages through HBM followed by stage 3 (LSB_NO_DYNFUSE=1): powers of two, lengths
+    with a factor 3 or 5 whose tiles are partial in x and y (nx = 96, ny = 30), a grid of
     four x tiles (these three with 4 planes per block and 65 planes, so the last block
     holds one) and a 512 x 129 x 256 grid with 16 planes per block, as at C4."""
     case = L.cases.CASES["c2_dyn_les"].with_(name=f"dyna{nx}x{ny}", nx=nx, ny=ny, nz=nz, dyn_avg=0, pert_rms=1e-2)
@@ -150,15 +150,15 @@ def test_mixed_dynamic_fused_average_bit_identical(nx, ny, nz, monkeypatch):
 
 
 @pytest.mark.parametrize("nx,ny,forcing", [(128, 64, 0), (96, 30, 1)])
-def test_mixed_dynamic_stage1_pairs_bit_identical(nx, ny, forcing, monkeypatch):
-    """Stages 1 and 2 of the mixed dynamic model with two x points per thread (8-byte loads
-    and stores) give the same bits as one point per thread (LSB_NO_DYNX2=1), with and
+def test_mixed_dynamic_stages_and_filter_bit_identical(nx, ny, forcing, monkeypatch):
+    """Stages 1 and 2 of the mixed dynamic model with the test filter between them in one pass
+    give the same bits as passes of their own (LSB_NO_DYNFUSE=1) over ten steps, with and
     without the sponge term."""
     case = L.cases.CASES["c2_dyn_les"].with_(name=f"dyn1x{nx}x{ny}", nx=nx, ny=ny, nz=64, dyn_avg=0, pert_rms=1e-2)
     u, v, w = L.cases.initial_condition(case)
     out = {}
     for single in ("0", "1"):
-        monkeypatch.setenv("LSB_NO_DYNX2", single)
+        monkeypatch.setenv("LSB_NO_DYNFUSE", single)
         c = setup_case(case, precision=1, forcing=forcing)
         try:
             if forcing:
@@ -171,7 +171,7 @@ def test_mixed_dynamic_stage1_pairs_bit_identical(nx, ny, forcing, monkeypatch):
     for k in VEL + ("pf", "nlnif", "nlnmif"):
         assert np.all(np.isfinite(out["0"][k])), k
         assert np.array_equal(out["0"][k], out["1"][k]), k
-    print("stages 1 and 2, two points per thread, bit-identical:", case.name, "forcing", forcing, flush=True)
+    print("stages 1 and 2 with the filter, bit-identical:", case.name, "forcing", forcing, flush=True)
 
 
 @pytest.mark.parametrize("dealias", [2, 0])
