@@ -327,17 +327,34 @@ __global__ void __launch_bounds__(64 * (R + 2)) k_dynm_test(DDims d, DynMixArgs<
     double za[21], zb[21];
 #pragma unroll
     for (int f = 0; f < 21; ++f) za[f] = zb[f] = 0.0;
-    for (int kk = kstart; kk <= klast; ++kk) {
+    auto ypass = [&](int f) {
+        return div(wa * xs[f][r - 1][lane] + wb * xs[f][r][lane] + wa * xs[f][r + 1][lane]);
+    };
+    // a boundary plane keeps its xy-filtered values (no z pass: an infinite neighbour times
+    // a weight of 0 would not leave it alone)
+    auto edge = [&](int k) {
+        T num, den;
+        dynm_stage2_math(A, d.nzp, k, [&](int f) { return (double)(T)zb[f]; }, num, den);
+        put(k, num, den);
+    };
+    int kk = kstart;
+    if (k0 == 0) {
+        xphase(0);
+#pragma unroll
+        for (int f = 0; f < 21; ++f) zb[f] = ypass(f);
+        edge(0);
+        __syncthreads();
+        kk = 1;
+    }
+    for (; kk <= klast; ++kk) {
         xphase(kk);
         // weights of plane kk - 1 (w0) and kk (w1) in the output plane kk and of kk in kk - 1
-        // (w2); a boundary plane keeps its value (weights 0, 1, 0)
-        const bool zin = kk - 1 > 0;  // the output plane kk - 1 is below nzp - 1
-        const bool end = kk == 0 || kk == d.nzp - 1;
-        const double w2 = zin ? is * w[2 * d.nzp + kk - 1] : 0.0;
-        const double w1 = end ? 1.0 : is * w[d.nzp + kk];
-        const double w0 = end ? 0.0 : is * w[kk];
+        // (w2)
+        const double w2 = is * w[2 * d.nzp + kk - 1];
+        const double w1 = is * w[d.nzp + kk];
+        const double w0 = is * w[kk];
         auto yz = [&](int f) {
-            const double y = div(wa * xs[f][r - 1][lane] + wb * xs[f][r][lane] + wa * xs[f][r + 1][lane]);
+            const double y = ypass(f);
             // z = za + w2 y, za = w0 zb + w1 y in the three-address form (the two-address one
             // costs copies of the sums on every plane)
             const double t = w1 * y;
@@ -345,20 +362,15 @@ __global__ void __launch_bounds__(64 * (R + 2)) k_dynm_test(DDims d, DynMixArgs<
             asm("v_fma_f64 %0, %1, %2, %3" : "=v"(z) : "s"(w2), "v"(y), "v"(za[f]));
             asm("v_fma_f64 %0, %1, %2, %3" : "=v"(za[f]) : "s"(w0), "v"(zb[f]), "v"(t));
             zb[f] = y;
-            if constexpr (!P2) z = zin ? z / s : z;
+            if constexpr (!P2) z = z / s;
             return (double)(T)z;
         };
         T num, den;
         dynm_stage2_math(A, d.nzp, max(kk - 1, 0), yz, num, den);
-        if (kk > k0) put(kk - 1, num, den);
+        if (kk > max(k0, 1)) put(kk - 1, num, den);
         __syncthreads();
     }
-    // the last plane of the grid keeps its xy-filtered value (no z pass)
-    if (k1 == d.nzp) {
-        T num, den;
-        dynm_stage2_math(A, d.nzp, d.nzp - 1, [&](int f) { return (double)(T)za[f]; }, num, den);
-        put(d.nzp - 1, num, den);
-    }
+    if (k1 == d.nzp) edge(d.nzp - 1);
 }
 
 // stage 3 at one point of plane k from the coefficient ratio ct = <M:L> / <M:M>
