@@ -74,8 +74,10 @@ def test_step_against_unfused(nx, ny, nz, monkeypatch):
 @pytest.mark.parametrize("sigma", [0.0, 2.0e5])
 def test_fp32_and_refined_solve(nx, ny, nz, sigma, monkeypatch):
     """The one-kernel solves against the FP64 solution: FP32's rounding times the solve's
-    conditioning (the separate kernels' error up to the order of its sums), and after the
-    refinement that error times itself, at least four digits below."""
+    conditioning (1.7e-7 at most here; the separate kernels' error up to the order of its
+    sums), and after the refinement that error times itself, at least four digits below.
+    The two routes sum in different orders, so equal bits would mean that one of them ran
+    twice."""
     hip = Hip()
     with setup_case(L.cases.CASES["c2_dyn_les"].with_(nx=nx, ny=ny, nz=nz)) as ctx:
         rhs = c3_rhs(nz + 1, nx * ny, 2).reshape(2, nz + 1, ny, nx)
@@ -87,4 +89,6 @@ def test_fp32_and_refined_solve(nx, ny, nz, sigma, monkeypatch):
     print(f"{nx}x{nz + 1}x{ny} sigma {sigma}: FP32 {e[0]:.1e} refined {e[1]:.1e}; separate {e[2]:.1e} {e[3]:.1e}",
           flush=True)
     assert np.all(ur[:, 0] == 0.0) and np.all(ur[:, nz] == 0.0) and np.all(u32[:, nz] == 0.0)
+    assert not np.array_equal(u32, s32) and not np.array_equal(ur, sr)
+    assert e[0] < 1e-6 and e[1] < 1e-4 * e[0]
     assert e[0] < 4.0 * e[2] and e[1] < 4.0 * max(e[3], 1e-15)
