@@ -222,7 +222,7 @@ def traffic_class(name):
 def pmc_summarize(fetch_csv, write_csv, out_path=TRAFFIC_FILE, steps_per_form=2):
     """HBM bytes per kernel and per class and step from the FETCH_SIZE and WRITE_SIZE runs of
     --pmc-probe: each counter scaled by what it reads for the 1 GiB copy; the FP64 form's
-    kernels are those up to its last step's final k_norm_nyq, the mixed form's follow."""
+    kernels are those up to its last step's final k_norm, the mixed form's follow."""
     import csv
 
     def load(fn, counter):
@@ -236,7 +236,7 @@ def pmc_summarize(fetch_csv, write_csv, out_path=TRAFFIC_FILE, steps_per_form=2)
     ci = next(i for i, (n, v) in enumerate(F) if "copyBuffer" in n and v > 1e5)
     fetch_cal = COPY_BYTES / (F[ci][1] * 1024.0)
     write_cal = COPY_BYTES / (W[ci][1] * 1024.0)
-    ends = [i for i, (n, _) in enumerate(F) if "k_norm_nyq" in n]
+    ends = [i for i, (n, _) in enumerate(F) if n == "lsb::k_norm"]
     last_fp64 = ends[steps_per_form - 1]
     out = {"sources_sha": sources_digest(),
            "calibration": {"copy_bytes": COPY_BYTES, "fetch_kib": F[ci][1], "write_kib": W[ci][1],

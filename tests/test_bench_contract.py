@@ -1,7 +1,11 @@
-"""bench.py's host logic on the CPU: the mixed-vs-FP64 comparison of two states, and the
-single-GPU refusal of --gpus above 1 (before anything touches a GPU)."""
+"""bench.py's host logic on the CPU: the mixed-vs-FP64 comparison of two states, the HBM-traffic
+table of two counter files, and the single-GPU refusal of --gpus above 1 (before anything
+touches a GPU)."""
 
+import csv
+import json
 import os
+import re
 import subprocess
 import sys
 
@@ -41,3 +45,31 @@ def test_several_gpus_refused():
                        text=True, timeout=120, cwd=ROOT)
     assert r.returncode == 2
     assert "one GPU" in r.stderr
+
+
+def test_traffic_table_of_counter_files(tmp_path):
+    """Two steps of each form as the counter runs list them: a calibrating copy, and each step
+    ended by the norm, by the name that its kernel has in the sources."""
+    with open(os.path.join(ROOT, "lsbflow_amd", "csrc", "spectral.hip")) as fh:
+        norm = re.search(r"__global__ void (k_norm\w*)\(", fh.read()).group(1)
+    step = {"fp64": "void lsb::k_yfwd_rhs<double, double, 16, 16, 16>(int)",
+            "mixed": "void lsb::k_yfwd_rhs<float, float, 16, 16, 16>(int)"}
+    names = ["__amd_rocclr_copyBuffer"]
+    for form in ("fp64", "mixed"):
+        names += 2 * [step[form], f"lsb::{norm}(lsb::FieldList<double>, int)"]
+    kib = bench.COPY_BYTES / 1024.0
+    files = []
+    for counter, copied in (("FETCH_SIZE", kib / 2), ("WRITE_SIZE", kib)):
+        files.append(str(tmp_path / f"{counter}.csv"))
+        with open(files[-1], "w", newline="") as fh:
+            w = csv.writer(fh)
+            w.writerow(["Dispatch_Id", "Kernel_Name", "Counter_Name", "Counter_Value"])
+            for i, n in enumerate(names):
+                v = copied if i == 0 else 100.0 if "double, double" in n else 50.0 if "float" in n else 1.0
+                w.writerow([i, n, counter, v])
+    out = str(tmp_path / "traffic.json")
+    assert bench.pmc_summarize(*files, out_path=out) == 0
+    with open(out) as fh:
+        t = json.load(fh)
+    assert t["classes"]["fp64"]["rhs"]["bytes_per_step"] == 100 * 1024 * 3
+    assert t["classes"]["mixed"]["rhs"]["bytes_per_step"] == 50 * 1024 * 3
