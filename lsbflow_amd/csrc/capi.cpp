@@ -281,10 +281,12 @@ extern "C" int lsb_create(const lsb_config* cfg, lsb_ctx** out) {
     }
     rc = hor_plan_create(&c->hp, c->nx, c->ny);
     // The mixed form without an SGS model keeps the Stockham passes at the lengths with a
-    // factor 3 or 5: its perturbation is small and its pressure, a divergence over k^2 dt,
-    // carries the FP32 rounding of the nonlinear chain at 1e-5 to 1e-4 of itself (against the
-    // FP64 form, with either transform), so another order of the transforms moves it by as
-    // much; under the ceiling of the LES it is 1e3 larger and the same change is below 1e-6.
+    // factor 3 or 5, so that its results stay to the bit what they were: its pressure, a
+    // divergence over k^2 dt, carries the FP32 rounding of the nonlinear chain at 2e-5 of
+    // itself with either transform (from the FP64 form, five steps without a ceiling), and
+    // another order of the transforms moves it by as much.  The rule is about stored results,
+    // not about accuracy: the LES take the register-resident passes at the same distance from
+    // the FP64 form as with the Stockham ones (2e-5 without a ceiling, 1e-8 to 9e-8 with it).
     c->hp.pow2_only = c->cfg.precision == LSB_MIXED && !(c->cfg.sgsflag == 1 && c->cfg.sgsmodel != 4);
     if (rc == LSB_OK) rc = upload_context(c);
     if (rc == LSB_OK) rc = noalloc_resolve(g.device);

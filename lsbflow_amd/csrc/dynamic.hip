@@ -240,11 +240,14 @@ __device__ __forceinline__ double lane_next(double v) {
 // (zb) and the sum over the last two (za) in registers, and stage 2.  The loads of
 // the next plane are in flight meanwhile.  The 21 values are rounded to T where the separate
 // passes store them, in their expressions: the same bits.
-// 14 field passes in place of 99; bound by the vector units (some 410 instructions per point
-// and plane, 4/3 of the x phase for the halo rows) with HBM close behind.  R = 6: 8 waves
-// with up to 256 registers (42 FP64 values of the z pass each); R = 4 and R = 10 leave 168 and spill (FP64
-// step at 512x193x256: 8.36 ms against 10.6 and 13.3).  At that grid 1.13 ms in place of
-// 1.62 + 2.08 + 0.94 for stage 1, the filter and stage 2.
+// 14 field passes in place of 99, and the halo: at 512x193x256 the FP64 form reads 4.3 GB
+// (12 fields are 2.5) and writes 0.4 in 1.10 ms, 4.3 TB/s, bound by HBM with the vector units
+// 0.4 busy; the mixed form moves 2.7 GB in 0.88 ms, 3.1 TB/s, the vector units 0.56 busy (some
+// 410 instructions per point and plane, 4/3 of the x phase for the halo rows), and waits at
+// two waves a SIMD.  R = 6: 8 waves with up to 256 registers (42 FP64 values of the z pass
+// each); R = 4 and R = 10 leave 168 and spill (FP64 step at that grid: 8.36 ms against 10.6
+// and 13.3).  The FP64 1.10 ms are in place of 1.62 + 2.08 + 0.94 for stage 1, the filter and
+// stage 2.
 template <class T, int R, bool P2>
 __global__ void __launch_bounds__(64 * (R + 2)) k_dynm_test(DDims d, DynMixArgs<T> A, const double* __restrict__ w,
                                                             double fa, double fb, int txo, int KC) {

@@ -576,7 +576,8 @@ int horfft_inv(lsb_ctx* c, const HorPlan& hp, const double* const* spec, double*
 }
 
 // ------------------------------------------- mixed form, generic lengths
-// Lengths that are not register-resident (fast_fft_len) run the mixed form's transforms on the Stockham kernels in FP32.
+// Lengths that are not register-resident (plan_fast) run the mixed form's transforms on the
+// Stockham kernels in FP32.
 
 // u, du/dx, du/dy of 3 FP64 spectra rounded to 9 FP32 spectra; the derivatives are
 // taken in FP64 first (derivatives.f90:261-303: i kx f, i ky f).  One thread per

@@ -670,9 +670,9 @@ __global__ void __launch_bounds__(C * N2) k_yinv3_fast(FieldList<TI> in, FieldLi
 // passes (nlt, then - i kx h_x, then - i ky h_y, each piece rounded to R after
 // scaling as the separate forward pass stores it): the results of fast_yfwd followed by the
 // right-hand-side kernel up to the last rounding of products that join a following sum.
-// HBM-bound: 30 FP64 field passes at some 5.3 TB/s where the two passes take 46; the FP64
-// step at 512x193x256 with the dynamic model 8.32 -> 7.74 ms, the 240x114x120 sigma step
-// 939 -> 885 us.
+// HBM-bound: 30 FP64 field passes (6.07 GB by the counters, 1.24 ms at 512x193x256: 4.9 TB/s)
+// where the two passes take 46; the FP64 step there with the dynamic model 8.32 -> 7.74 ms,
+// the 240x114x120 sigma step 939 -> 885 us.
 template <class TN>
 __device__ __forceinline__ void ld_h(const void* p, long q, double& re, double& im) {
     const TN* t = reinterpret_cast<const TN*>(p) + 2 * q;

@@ -287,8 +287,8 @@ __global__ void k_rhs_vel(SpDims d, const double* __restrict__ wavx, const doubl
 // planes.  One launch for three (the two-row contraction, which the matrix kernel ran on
 // tiles of 64 rows, the bound scaling and this): bound by reading w once, with 8 loads a
 // thread in flight on 16 modes a block so that small planes fill the chip too.  68 + 5 + 7 us
-// before at 512x193x256, 28 + 5 + 6 at 240x114x120; four 64x65x32 DNS steps 452 -> 394 us
-// with it and the one-launch norm.
+// before at 512x193x256 (now 56: 0.22 GB at 3.9 TB/s), 28 + 5 + 6 at 240x114x120 (now 12);
+// four 64x65x32 DNS steps 452 -> 394 us with it and the one-launch norm.
 constexpr int kBcPairs = 16;
 constexpr int kBcGroups = 16;
 constexpr int kBcPlanes = 128;

@@ -1530,9 +1530,9 @@ __device__ __forceinline__ void ztile_mul(V (&accE)[RB][CB], V (&accO)[RB][CB], 
 // the residual r - (D2 - k^2 - sigma) u (D2 parity-split, FP64 products) goes back into the
 // FP32 tile for the second solve; u += du at the store.  The separate kernels moved 22
 // field passes through HBM and bound the refined solve there; this one reads the
-// right-hand side twice (the second time from cache) and writes once: three fields of
-// 256x129x128 refined in 130 us against 690 (without the caller's copy), its error against
-// a 64-bit solution 3.0e-14 against 5.7e-14.
+// right-hand side twice (the second time from cache) and writes once: a caller's copy and
+// refined solve of three fields of 256x129x128 take 175 us against 740 (the kernel 153 us in
+// a trace), the error against a 64-bit solution 3.0e-14 against 5.7e-14.
 struct ZRefineArgs {
     const float *H1p, *H1q, *H2p, *H2q;  // Einv, E halves
     const double *Dp, *Dq;               // D2 halves (REFINE)
