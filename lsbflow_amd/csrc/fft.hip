@@ -515,9 +515,9 @@ int horfft_inv_ops(lsb_ctx* c, const HorPlan& hp, const double* const* spec, dou
         prof_mark_end(c, tok, s);
         return LSB_OK;
     }
-    if (horfft_has_ops(hp)) {
-        const size_t splane = (size_t)nx * ny, pplane = (size_t)nxpp * ny;
-        const int budget = (int)std::clamp<size_t>(kInvPiece / (pplane * sizeof(double)), 1, 1 << 20);  // planes
+    const size_t splane = (size_t)nx * ny, pplane = (size_t)nxpp * ny;
+    const int budget = (int)std::clamp<size_t>(kInvPiece / (pplane * sizeof(double)), 1, 1 << 20);  // planes
+    if (horfft_has_ops(hp) && (long)nf * nplanes > budget) {
         // pieces of whole fields, or of one field's planes; the first ones are the smaller
         const int kp = (nplanes + budget - 1) / budget;
         const int fp = kp > 1 ? nf : (nf + budget / nplanes - 1) / (budget / nplanes);
